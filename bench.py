@@ -10,7 +10,11 @@ results bit for bit.  A "step" is one collide-stream iteration of the
 whole lattice.  The timed region
 holds exactly --steps iterations enqueued back to back on the library's stream,
 bracketed by device synchronisation; the lattice is resident in HBM and already
-initialised before it starts.
+initialised before it starts.  Without per-launch events the library advances
+two iterations per launch where the lattice has such a kernel (native storage
+from 128^3 on): `value`, `mlups` and `ms_per_step` are of those; with events
+every iteration is a launch of its own, which is what `kernel_mlups` and the
+roofline time.
 
 Printed: one JSON line with MLUPS (the reference's definition,
 (dim-2)^3 * iterations / time, lbmcl.hpp:601-620), the HBM roofline of the

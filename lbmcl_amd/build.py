@@ -16,6 +16,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -48,16 +49,27 @@ def _run(cmd):
 OBJ_DIR = os.path.join(PKG, "_build")
 
 
+# Units of liblbm_hip.so, and the flags a unit needs beyond HIP_FLAGS: the
+# LBM_ARITH_OPENCL kernels need OpenCL's FP32 division precision.
+OPENCL_DIVISION = ["-fno-hip-fp32-correctly-rounded-divide-sqrt"]
+LIB_UNITS = {
+    "lbm_capi": [], "lbm_adjoint": [], "lbm_noalloc": [], "lbm_two_step": [],
+    "lbm_opencl_arith": OPENCL_DIVISION, "lbm_two_step_opencl": OPENCL_DIVISION,
+}
+
+
 def build_lib():
-    # The LBM_ARITH_OPENCL kernels need OpenCL's FP32 division precision, a
-    # per-translation-unit flag: that unit is compiled on its own.
     os.makedirs(OBJ_DIR, exist_ok=True)
-    opencl_obj = os.path.join(OBJ_DIR, "lbm_opencl_arith.o")
-    _run([HIPCC, *HIP_FLAGS, "-fno-hip-fp32-correctly-rounded-divide-sqrt", "-c", "-I", INCLUDE, "-I", CSRC,
-          os.path.join(CSRC, "lbm_opencl_arith.hip"), "-o", opencl_obj])
-    _run([HIPCC, *HIP_FLAGS, "-shared", "-I", INCLUDE, "-I", CSRC,
-          os.path.join(CSRC, "lbm_capi.hip"), os.path.join(CSRC, "lbm_adjoint.hip"), os.path.join(CSRC, "lbm_noalloc.hip"),
-          "-x", "none", opencl_obj, "-o", LIB])
+
+    def compile_unit(unit):
+        obj = os.path.join(OBJ_DIR, unit + ".o")
+        _run([HIPCC, *HIP_FLAGS, *LIB_UNITS[unit], "-c", "-I", INCLUDE, "-I", CSRC,
+              os.path.join(CSRC, unit + ".hip"), "-o", obj])
+        return obj
+
+    with ThreadPoolExecutor(4) as pool:
+        objs = list(pool.map(compile_unit, LIB_UNITS))
+    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", *objs, "-o", LIB])
 
 
 def build_membw():

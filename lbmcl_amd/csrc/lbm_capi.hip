@@ -22,6 +22,28 @@ int enqueue_view(lbm_ctx* c, int32_t buffer, void* out, int64_t out_stride) {
     return launch_view<float, lbm::ST_NATIVE>(c, c->lat[buffer], static_cast<float*>(out), out_stride);
 }
 
+template <class T, int KIND> int launch_check_walls(lbm_ctx* c, const void* lattice, uint32_t* differ) {
+    const lbm::InitArgs<T> a = init_args<T, KIND>(c);
+    const int64_t nb = (c->n3 + 255) / 256;
+    hipLaunchKernelGGL((lbm::lbm_check_walls_kernel<T, KIND>), dim3(unsigned(nb)), dim3(256), 0, c->stream, a, lattice,
+                       differ);
+    LBM_HIP_CHECK(hipGetLastError(), "wall check launch");
+    return LBM_OK;
+}
+
+// Whether the wall cells of lattice `buffer` hold the initial lattice's values.
+int check_walls(lbm_ctx* c, int32_t buffer, bool* same) {
+    uint32_t* differ = reinterpret_cast<uint32_t*>(c->partials);  // free between launches that reduce
+    LBM_HIP_CHECK(hipMemsetAsync(differ, 0, sizeof *differ, c->stream), "hipMemsetAsync");
+    const int rc = LBM_DISPATCH(c, launch_check_walls, c, static_cast<const void*>(c->lat[buffer]), differ);
+    if (rc) return rc;
+    uint32_t h = 1;
+    LBM_HIP_CHECK(hipMemcpyAsync(&h, differ, sizeof h, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync D2H");
+    LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    *same = h == 0;
+    return LBM_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -123,6 +145,7 @@ int lbm_initialize(lbm_ctx* c) {
     rc = ev_end(c, r);
     if (rc) return rc;
     c->initialized = true;
+    c->walls_initial[0] = c->walls_initial[1] = true;
     c->diag_valid = false;
     return LBM_OK;
 }
@@ -163,10 +186,26 @@ int lbm_compute_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
     LBM_CHECK_CTX(c);
     LBM_CHECK_INIT(c);
     if (first < 1 || count < 0 || every < 0) return fail(LBM_ERR_INVALID, "bad iteration range");
-    for (int64_t it = first; it < first + count; ++it) {
-        const int um = (every > 0 && it % every == 0) ? 1 : 0;
-        const int rc = lbm_compute(c, it, um, 0);
+    // Without per-launch events, two iterations go in one launch where the
+    // lattice has one (lbm_two_step.hpp).  The iteration in between reaches no
+    // lattice, so the last one is always a launch of its own -- it leaves the last
+    // two states in the two lattices, as iterations one by one do -- and so is one
+    // that stores rho and u and is not the second of its pair.
+    const bool pairs = !c->cfg.profile && c->walls_initial[0] && c->walls_initial[1] && two_steps_preferred(c);
+    const int64_t end = first + count;
+    for (int64_t it = first; it < end;) {
+        const auto stores = [&](int64_t k) { return every > 0 && k % every == 0 ? 1 : 0; };
+        if (pairs && end - it >= 3 && !stores(it)) {
+            const int s = (it % 2 != 0) ? 0 : 1;
+            const int rc = launch_two_steps(c, c->lat[s], c->lat[1 - s], stores(it + 1));
+            if (rc) return rc;
+            std::swap(c->lat[0], c->lat[1]);  // iteration it + 2 reads the lattice just written, as lattice s again
+            it += 2;
+            continue;
+        }
+        const int rc = lbm_compute(c, it, stores(it), 0);
         if (rc) return rc;
+        ++it;
     }
     return LBM_OK;
 }
@@ -350,9 +389,14 @@ int lbm_write_state(lbm_ctx* c, int32_t buffer, const void* in) {
     LBM_CHECK_INIT(c);
     if (!in) return fail(LBM_ERR_INVALID, "null input");
     if (buffer != 0 && buffer != 1) return fail(LBM_ERR_INVALID, "buffer must be 0 or 1");
+    c->walls_initial[buffer] = false;
     LBM_HIP_CHECK(hipMemcpyAsync(c->lat[buffer], in, size_t(c->n3) * lbm::Q * c->ssize, hipMemcpyHostToDevice,
                                  c->stream),
                   "hipMemcpyAsync H2D");
+    if (two_steps_possible(c)) {
+        const int rc = check_walls(c, buffer, &c->walls_initial[buffer]);
+        if (rc) return rc;
+    }
     LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     return LBM_OK;
 }

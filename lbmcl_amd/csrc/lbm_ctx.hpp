@@ -124,6 +124,9 @@ struct StepPlan {
 
 struct lbm_ctx : lbm_host::StepPlan {
     void* lat[2] = {nullptr, nullptr};  // lat[0] read by odd iterations, lat[1] by even
+    // whether the wall cells' slots of each lattice hold the initial lattice's
+    // values: so from lbm_initialize on, unless lbm_write_state brought others
+    bool walls_initial[2] = {false, false};
     int32_t* map = nullptr;      // cell flags, allocated on first read (ensure_map)
     bool map_valid = false;
     int64_t partials_cap = 0;  // in blocks
@@ -474,6 +477,15 @@ inline int plan_from_config(const lbm_config& k, StepPlan* p) {
     return LBM_OK;
 }
 
+// Two iterations in one launch (lbm_two_step.hpp), defined in lbm_two_step.hip:
+// whether AUTO takes it for the plan's lattice, whatever its force, and with the
+// force it has now; and the launch itself (macro_last: store rho and u of the
+// second iteration).  The wall cells of both lattices have to hold their initial
+// values.
+bool two_steps_possible(const StepPlan* c);
+bool two_steps_preferred(const StepPlan* c);
+int launch_two_steps(StepPlan* c, const void* src, void* dst, int macro_last);
+
 // Compute launches in the OpenCL arithmetic form, defined in
 // lbm_opencl_arith.hip (built with OpenCL's FP32 division precision).
 int launch_compute_opencl_f32(StepPlan* c, const void* src, void* dst, int update_macro, int diag, hipEvent_t e0,
@@ -507,9 +519,9 @@ inline size_t small_lattice_lds_pad(const StepPlan* c, unsigned block_threads) {
     return size_t(160 * 1024) / blocks_per_cu - 2048;
 }
 
-template <class T, int KIND, int ARITH>
-inline int launch_compute_impl(StepPlan* c, const void* src, void* dst, int update_macro, int diag, hipEvent_t e0,
-                               hipEvent_t e1) {
+// The arguments that every compute kernel takes from the plan.
+template <class T, int ARITH>
+inline lbm::StepArgs<T> step_args(const StepPlan* c, const void* src, void* dst, int update_macro, int diag) {
     lbm::StepArgs<T> a{};
     a.src = src;
     a.dst = dst;
@@ -546,6 +558,13 @@ inline int launch_compute_impl(StepPlan* c, const void* src, void* dst, int upda
             for (int i = 0; i < lbm::Q; ++i) a.lid_eq[i] = lbm::feq<T>(i, T(1), U, T(0), T(0), u2);
         }
     }
+    return a;
+}
+
+template <class T, int KIND, int ARITH>
+inline int launch_compute_impl(StepPlan* c, const void* src, void* dst, int update_macro, int diag, hipEvent_t e0,
+                               hipEvent_t e1) {
+    lbm::StepArgs<T> a = step_args<T, ARITH>(c, src, dst, update_macro, diag);
     const KernelKind kk = kernel_kind(c);
     if (kk == K_LDS) {
         const dim3 grid(unsigned(lds_grid(c->n, int64_t(c->ssize))));
@@ -616,7 +635,7 @@ inline int launch_compute(StepPlan* c, const void* src, void* dst, int update_ma
 }
 
 template <class T, int KIND>
-inline int launch_initialize(lbm_ctx* c) {
+inline lbm::InitArgs<T> init_args(const lbm_ctx* c) {
     lbm::InitArgs<T> a{};
     a.a = c->lat[0];
     a.b = c->lat[1];
@@ -635,6 +654,12 @@ inline int launch_initialize(lbm_ctx* c) {
         lbm::delta_lid_initial(float(c->U), d);
         for (int i = 0; i < lbm::Q; ++i) a.lid_delta[i] = T(d[i]);
     }
+    return a;
+}
+
+template <class T, int KIND>
+inline int launch_initialize(lbm_ctx* c) {
+    const lbm::InitArgs<T> a = init_args<T, KIND>(c);
     const int64_t nb = (c->n3 + 255) / 256;
     hipLaunchKernelGGL((lbm::lbm_initialize_kernel<T, KIND>), dim3(unsigned(nb)), dim3(256), 0, c->stream, a);
     LBM_HIP_CHECK(hipGetLastError(), "initialize launch");

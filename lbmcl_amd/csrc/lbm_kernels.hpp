@@ -1377,11 +1377,36 @@ template <class T> struct InitArgs {
     T lid_delta[Q];      // 16-bit storage (deviation form): F0 - w_i of FRONT cells
 };
 
+// P0[s][i] of cell s = (x, y, z), as stored
+template <class T, int KIND>
+__device__ __forceinline__ typename Codec<T, KIND>::S initial_slot(const InitArgs<T>& a, int i, int32_t x, int32_t y,
+                                                                   int32_t z) {
+    const Codec<T, KIND> codec{a.scale, a.inv_scale};
+    const int32_t n = a.n;
+    const int32_t dx = x + ex_of(i), dy = y + ey_of(i), dz = z + ez_of(i);
+    T v = __builtin_nan("");
+    if (dx >= 0 && dy >= 0 && dz >= 0 && dx < n && dy < n && dz < n) {
+        const int32_t td = cell_type(dx, dy, dz, n);
+        if (!is_wall(td) && KIND != ST_NATIVE) {
+            v = is_moving_init(td) ? a.lid_delta[i] : T(0);  // deviation form
+        } else if (!is_wall(td)) {
+            // kernels.cl:292-308 with rho = 1, u = (U or 0, 0, 0)
+            const T ux = is_moving_init(td) ? a.U : T(0);
+            if (a.contracted) {
+                v = feq_contracted<T>(i, T(1), ux, T(0), T(0), u2_contracted<T>(ux, T(0), T(0)));
+            } else {
+                const T u2 = ((ux * ux) + (T(0) * T(0))) + (T(0) * T(0));
+                v = feq<T>(i, T(1), ux, T(0), T(0), u2);
+            }
+        }
+    }
+    if constexpr (KIND != ST_NATIVE) return codec.encode_delta(v);
+    else return v;
+}
+
 template <class T, int KIND>
 __global__ __launch_bounds__(256) void lbm_initialize_kernel(InitArgs<T> a) {
-    using C = Codec<T, KIND>;
-    using S = typename C::S;
-    const C codec{a.scale, a.inv_scale};
+    using S = typename Codec<T, KIND>::S;
     const int32_t n = a.n;
     const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= a.n3) return;
@@ -1399,33 +1424,36 @@ __global__ __launch_bounds__(256) void lbm_initialize_kernel(InitArgs<T> a) {
     S* pb = static_cast<S*>(a.b);
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-        const int32_t dx = x + ex_of(i), dy = y + ey_of(i), dz = z + ez_of(i);
-        T v = qnan;
-        if (dx >= 0 && dy >= 0 && dz >= 0 && dx < n && dy < n && dz < n) {
-            const int32_t td = cell_type(dx, dy, dz, n);
-            if (!is_wall(td) && KIND != ST_NATIVE) {
-                v = is_moving_init(td) ? a.lid_delta[i] : T(0);  // deviation form
-            } else if (!is_wall(td)) {
-                // kernels.cl:292-308 with rho = 1, u = (U or 0, 0, 0)
-                const T ux = is_moving_init(td) ? a.U : T(0);
-                if (a.contracted) {
-                    v = feq_contracted<T>(i, T(1), ux, T(0), T(0), u2_contracted<T>(ux, T(0), T(0)));
-                } else {
-                    const T u2 = ((ux * ux) + (T(0) * T(0))) + (T(0) * T(0));
-                    v = feq<T>(i, T(1), ux, T(0), T(0), u2);
-                }
-            }
-        }
+        const S h = initial_slot<T, KIND>(a, i, x, y, z);
         const int64_t s = slot(c, i, a.stride);
-        if constexpr (KIND != ST_NATIVE) {
-            const S h = codec.encode_delta(v);
-            __builtin_nontemporal_store(h, pa + s);
-            __builtin_nontemporal_store(h, pb + s);
-        } else {
-            codec.store(pa + s, w_of<T>(i), v);
-            codec.store(pb + s, w_of<T>(i), v);
-        }
+        __builtin_nontemporal_store(h, pa + s);
+        __builtin_nontemporal_store(h, pb + s);
     }
+}
+
+// *differ = 1 where a wall cell's slot does not hold its initial value (a NaN
+// stands for any NaN).
+template <class T, int KIND>
+__global__ __launch_bounds__(256) void lbm_check_walls_kernel(InitArgs<T> a, const void* lattice, uint32_t* differ) {
+    using S = typename Codec<T, KIND>::S;
+    using U = typename std::conditional<sizeof(S) == 8, uint64_t,
+                                        typename std::conditional<sizeof(S) == 4, uint32_t, uint16_t>::type>::type;
+    const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (c >= a.n3) return;
+    const int32_t x = int32_t(c & (a.n - 1));
+    const int32_t y = int32_t((c >> a.log2n) & (a.n - 1));
+    const int32_t z = int32_t(c >> (2 * a.log2n));
+    if (!is_wall(cell_type(x, y, z, a.n))) return;
+    const Codec<T, KIND> codec{a.scale, a.inv_scale};
+    const S* p = static_cast<const S*>(lattice);
+    bool same = true;
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        const S want = initial_slot<T, KIND>(a, i, x, y, z), have = p[slot(c, i, a.stride)];
+        const T w = codec.decode(want, T(0)), h = codec.decode(have, T(0));
+        same = same && (__builtin_bit_cast(U, want) == __builtin_bit_cast(U, have) || (w != w && h != h));
+    }
+    if (!same) *differ = 1;
 }
 
 // The cell flags (common.h:7-20), materialised only when a caller reads the
