@@ -53,8 +53,9 @@ OBJ_DIR = os.path.join(PKG, "_build")
 # LBM_ARITH_OPENCL kernels need OpenCL's FP32 division precision.
 OPENCL_DIVISION = ["-fno-hip-fp32-correctly-rounded-divide-sqrt"]
 LIB_UNITS = {
-    "lbm_capi": [], "lbm_adjoint": [], "lbm_noalloc": [], "lbm_two_step": [],
+    "lbm_capi": [], "lbm_adjoint": [], "lbm_noalloc": [], "lbm_two_step": [], "lbm_small": [],
     "lbm_opencl_arith": OPENCL_DIVISION, "lbm_two_step_opencl": OPENCL_DIVISION,
+    "lbm_small_opencl": OPENCL_DIVISION,
 }
 
 
@@ -67,7 +68,7 @@ def build_lib():
               os.path.join(CSRC, unit + ".hip"), "-o", obj])
         return obj
 
-    with ThreadPoolExecutor(4) as pool:
+    with ThreadPoolExecutor(8) as pool:
         objs = list(pool.map(compile_unit, LIB_UNITS))
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", *objs, "-o", LIB])
 

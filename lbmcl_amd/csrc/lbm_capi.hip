@@ -5,6 +5,7 @@
 // the place of the OpenCL device layer of LBMCL (lbmcl.hpp:392-593,
 // libs/CLUtil.hpp).
 #include "lbm_ctx.hpp"
+#include "lbm_range.hpp"
 
 using namespace lbm_host;
 
@@ -186,26 +187,38 @@ int lbm_compute_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
     LBM_CHECK_CTX(c);
     LBM_CHECK_INIT(c);
     if (first < 1 || count < 0 || every < 0) return fail(LBM_ERR_INVALID, "bad iteration range");
-    // Without per-launch events, two iterations go in one launch where the
-    // lattice has one (lbm_two_step.hpp).  The iteration in between reaches no
-    // lattice, so the last one is always a launch of its own -- it leaves the last
-    // two states in the two lattices, as iterations one by one do -- and so is one
-    // that stores rho and u and is not the second of its pair.
-    const bool pairs = !c->cfg.profile && c->walls_initial[0] && c->walls_initial[1] && two_steps_preferred(c);
+    // Without per-launch events, several iterations go in one launch where the
+    // lattice has one (lbm_small.hpp, lbm_two_step.hpp).  Those in between reach
+    // no lattice, so the last one is a launch of its own -- it leaves the last two
+    // states in the two lattices, as iterations one by one do -- except where the
+    // launch itself does that.  The two-step launch stores rho and u of its second
+    // iteration only.
+    const bool multi = !c->cfg.profile && c->walls_initial[0] && c->walls_initial[1];
+    const int32_t small = multi ? small_steps(c) : 0;
+    const bool pairs = multi && !small && two_steps_preferred(c);
     const int64_t end = first + count;
     for (int64_t it = first; it < end;) {
         const auto stores = [&](int64_t k) { return every > 0 && k % every == 0 ? 1 : 0; };
-        if (pairs && end - it >= 3 && !stores(it)) {
-            const int s = (it % 2 != 0) ? 0 : 1;
-            const int rc = launch_two_steps(c, c->lat[s], c->lat[1 - s], stores(it + 1));
-            if (rc) return rc;
-            std::swap(c->lat[0], c->lat[1]);  // iteration it + 2 reads the lattice just written, as lattice s again
-            it += 2;
-            continue;
+        const int s = (it % 2 != 0) ? 0 : 1;  // the lattice that iteration `it` reads
+        int64_t k = 1;
+        int rc = LBM_OK;
+        if (small && small_is_one_tile(c)) {
+            k = std::min<int64_t>(small, end - it);
+            rc = launch_small(c, c->lat[s], c->lat[(s + k) % 2], k > 1 ? c->lat[(s + k + 1) % 2] : nullptr, int32_t(k),
+                              every, every > 0 ? (it - 1) % every : 0);
+        } else if (small && end - it >= 3) {
+            k = std::min<int64_t>(small, end - it - 1);
+            rc = launch_small(c, c->lat[s], c->lat[1 - s], nullptr, int32_t(k), every, every > 0 ? (it - 1) % every : 0);
+            if (!rc && k % 2 == 0) std::swap(c->lat[0], c->lat[1]);  // the lattice written is the one `it` + k reads
+        } else if (pairs && end - it >= 3 && !stores(it)) {
+            k = 2;
+            rc = launch_two_steps(c, c->lat[s], c->lat[1 - s], stores(it + 1));
+            if (!rc) std::swap(c->lat[0], c->lat[1]);
+        } else {
+            rc = lbm_compute(c, it, stores(it), 0);
         }
-        const int rc = lbm_compute(c, it, stores(it), 0);
         if (rc) return rc;
-        ++it;
+        it += k;
     }
     return LBM_OK;
 }
@@ -393,7 +406,7 @@ int lbm_write_state(lbm_ctx* c, int32_t buffer, const void* in) {
     LBM_HIP_CHECK(hipMemcpyAsync(c->lat[buffer], in, size_t(c->n3) * lbm::Q * c->ssize, hipMemcpyHostToDevice,
                                  c->stream),
                   "hipMemcpyAsync H2D");
-    if (two_steps_possible(c)) {
+    if (two_steps_possible(c) || small_steps(c)) {
         const int rc = check_walls(c, buffer, &c->walls_initial[buffer]);
         if (rc) return rc;
     }
