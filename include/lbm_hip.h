@@ -330,6 +330,10 @@ int lbm_adjoint(lbm_ctx* ctx, const lbm_adjoint_config* config, lbm_adjoint_resu
 int lbm_compute_noalloc(const lbm_config* cfg, const void* src, void* dst, void* rho, void* u, int32_t update_macro,
                         double* diag, void* stream);
 
+/* Give back what the library keeps between contexts: the pinned buffers of
+ * blocking reads (32 MiB at most).  They are allocated again when needed. */
+int lbm_trim(void);
+
 /* Text of the calling thread's last error ("" if none). */
 const char* lbm_last_error(void);
 

@@ -44,7 +44,7 @@ EXPORTS = (
     "lbm_read_f", "lbm_read_state", "lbm_write_state", "lbm_read_diagnostics", "lbm_get_constants",
     "lbm_event_count", "lbm_event_get", "lbm_total_time_ms", "lbm_kernels_time_ms", "lbm_clear_events",
     "lbm_set_force", "lbm_adjoint", "lbm_snapshot", "lbm_snapshot_wait", "lbm_snapshot_release", "lbm_last_error",
-    "lbm_compute_noalloc",
+    "lbm_compute_noalloc", "lbm_trim",
 )
 
 LBM_SNAPSHOT_MACRO, LBM_SNAPSHOT_F, LBM_SNAPSHOT_MAP = 0, 1, 2
@@ -148,6 +148,7 @@ def _declare(L):
         "lbm_snapshot_wait": [vp, i64, P(vp), P(i64)],
         "lbm_snapshot_release": [vp, i64],
         "lbm_compute_noalloc": [P(LbmConfig), vp, vp, vp, vp, i32, vp, vp],
+        "lbm_trim": [],
     }
     for name, args in sig.items():
         fn = getattr(L, name)
@@ -176,6 +177,11 @@ def device_name(device=0) -> str:
     buf = ctypes.create_string_buffer(256)
     check(lib().lbm_get_device_name(device, buf, 256), "lbm_get_device_name")
     return buf.value.decode()
+
+
+def trim():
+    """Give back what the library keeps between contexts (lbm_trim)."""
+    check(lib().lbm_trim(), "lbm_trim")
 
 
 def _ptr(a: np.ndarray):

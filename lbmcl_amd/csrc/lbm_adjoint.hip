@@ -233,12 +233,9 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     LBM_HIP_CHECK(hipEventRecord(e2, c->stream), "hipEventRecord");
 
     double h[3];
-    LBM_HIP_CHECK(hipMemcpyAsync(h, acc, sizeof h, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync D2H");
-    if (grad_g_host)
-        LBM_HIP_CHECK(hipMemcpyAsync(grad_g_host, grad_g, size_t(3 * c->n3) * sizeof(double), hipMemcpyDeviceToHost,
-                                     c->stream),
-                      "hipMemcpyAsync D2H");
-    LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    rc = copy_to_host(c, h, acc, sizeof h);
+    if (!rc && grad_g_host) rc = copy_to_host(c, grad_g_host, grad_g, size_t(3 * c->n3) * sizeof(double));
+    if (rc) return rc;
     float fms = 0.f, ams = 0.f;
     LBM_HIP_CHECK(hipEventElapsedTime(&fms, e0, e1), "hipEventElapsedTime");
     LBM_HIP_CHECK(hipEventElapsedTime(&ams, e1, e2), "hipEventElapsedTime");

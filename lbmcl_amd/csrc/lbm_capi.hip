@@ -36,13 +36,12 @@ template <class T, int KIND> int launch_check_walls(lbm_ctx* c, const void* latt
 int check_walls(lbm_ctx* c, int32_t buffer, bool* same) {
     uint32_t* differ = reinterpret_cast<uint32_t*>(c->partials);  // free between launches that reduce
     LBM_HIP_CHECK(hipMemsetAsync(differ, 0, sizeof *differ, c->stream), "hipMemsetAsync");
-    const int rc = LBM_DISPATCH(c, launch_check_walls, c, static_cast<const void*>(c->lat[buffer]), differ);
+    int rc = LBM_DISPATCH(c, launch_check_walls, c, static_cast<const void*>(c->lat[buffer]), differ);
     if (rc) return rc;
     uint32_t h = 1;
-    LBM_HIP_CHECK(hipMemcpyAsync(&h, differ, sizeof h, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync D2H");
-    LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    *same = h == 0;
-    return LBM_OK;
+    rc = copy_to_host(c, &h, differ, sizeof h);
+    *same = !rc && h == 0;
+    return rc;
 }
 
 }  // namespace
@@ -237,11 +236,7 @@ int lbm_read_map(lbm_ctx* c, int32_t* out) {
     int rc = ev_begin(c, LBM_EVENT_READ_MAP, r);
     if (!rc) rc = ensure_map(c);
     if (rc) return rc;
-    LBM_HIP_CHECK(hipMemcpyAsync(out, c->map, size_t(c->n3) * 4, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync D2H");
-    rc = ev_end(c, r);
-    if (rc) return rc;
-    LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    return LBM_OK;
+    return copy_to_host(c, out, c->map, size_t(c->n3) * 4, &r);
 }
 
 int lbm_read_rho(lbm_ctx* c, void* out) {
@@ -270,11 +265,7 @@ int lbm_read_f(lbm_ctx* c, int32_t buffer, void* out) {
     EventRec r;
     rc = ev_begin(c, LBM_EVENT_READ_F, r);
     if (!rc) rc = enqueue_view(c, buffer, tmp, c->stride);
-    if (!rc) {
-        const hipError_t e = hipMemcpyAsync(out, tmp, bytes, hipMemcpyDeviceToHost, c->stream);
-        if (e != hipSuccess) rc = fail(LBM_ERR_RUNTIME, std::string("hipMemcpyAsync D2H: ") + hipGetErrorString(e));
-    }
-    if (!rc) rc = ev_end(c, r);
+    if (!rc) rc = copy_to_host(c, out, tmp, bytes, &r);
     const hipError_t se = hipStreamSynchronize(c->stream);
     (void)hipFree(tmp);
     if (rc) return rc;
@@ -419,8 +410,8 @@ int lbm_read_diagnostics(lbm_ctx* c, double* mass, double* kinetic_energy) {
     if (!mass || !kinetic_energy) return fail(LBM_ERR_INVALID, "null output");
     if (!c->diag_valid) return fail(LBM_ERR_STATE, "no compute with diagnostics enqueued");
     double h[2];
-    LBM_HIP_CHECK(hipMemcpyAsync(h, c->diag, sizeof h, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync D2H");
-    LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    const int rc = copy_to_host(c, h, c->diag, sizeof h);
+    if (rc) return rc;
     *mass = h[0];
     *kinetic_energy = h[1];
     return LBM_OK;
@@ -488,6 +479,12 @@ int lbm_kernels_time_ms(lbm_ctx* c, double* ms) {
         total += double(t);
     }
     *ms = total;
+    return LBM_OK;
+}
+
+int lbm_trim(void) {
+    std::lock_guard<std::mutex> lock(g_pinned.busy);
+    g_pinned.free();
     return LBM_OK;
 }
 

@@ -22,6 +22,7 @@
 #include "../../include/lbm_hip.h"
 #include "lbm_kernels.hpp"
 #include "lbm_slots.hpp"
+#include "lbm_stage.hpp"
 
 namespace lbm_host {
 
@@ -133,6 +134,7 @@ struct lbm_ctx : lbm_host::StepPlan {
     double* diag = nullptr;    // 2 doubles
     bool diag_valid = false;
     bool initialized = false;
+    lbm_host::HostStage stage;  // of blocking reads
     lbm_host::EventLog events;
     // asynchronous snapshots: staging slots and their state machine
     hipStream_t copy_stream = nullptr;
@@ -237,6 +239,7 @@ inline void release(lbm_ctx* c) {
         if (s.packed) (void)hipEventDestroy(s.packed);
     }
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
+    c->stage.release();
     free_events(c);
     for (void* p : {c->lat[0], c->lat[1], c->rho, c->u, (void*)c->map, (void*)c->partials, (void*)c->diag, c->force})
         if (p) (void)hipFree(p);
@@ -691,15 +694,21 @@ inline int launch_view(lbm_ctx* c, const void* p, T* out, int64_t out_stride) {
      : (c)->cfg.storage == LBM_STORE_BF16_SHIFT ? FN<float, lbm::ST_BF16>(__VA_ARGS__)  \
                                                 : FN<float, lbm::ST_NATIVE>(__VA_ARGS__))
 
+// Blocking copy of device memory into caller memory; the stop of `r` (null:
+// none) is recorded behind the last copy.
+inline int copy_to_host(lbm_ctx* c, void* dst, const void* src, size_t bytes, EventRec* r = nullptr) {
+    int rc = LBM_OK;
+    const hipError_t e = c->stage.copy(c->cfg.device, c->stream, dst, src, bytes, [&] {
+        if (r) rc = ev_end(c, *r);
+    });
+    if (e != hipSuccess) return fail(LBM_ERR_RUNTIME, std::string("copy to the host: ") + hipGetErrorString(e));
+    return rc;
+}
+
 inline int read_device(lbm_ctx* c, int kind, void* dst, const void* src, size_t bytes) {
     EventRec r;
-    int rc = ev_begin(c, kind, r);
-    if (rc) return rc;
-    LBM_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync D2H");
-    rc = ev_end(c, r);
-    if (rc) return rc;
-    LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    return LBM_OK;
+    const int rc = ev_begin(c, kind, r);
+    return rc ? rc : copy_to_host(c, dst, src, bytes, &r);
 }
 
 // The map buffer, allocated and filled on first use (lbm_read_map, map
