@@ -331,7 +331,10 @@ int lbm_compute_noalloc(const lbm_config* cfg, const void* src, void* dst, void*
                         double* diag, void* stream);
 
 /* Give back what the library keeps between contexts: the pinned buffers of
- * blocking reads (32 MiB at most).  They are allocated again when needed. */
+ * blocking reads (32 MiB at most) and the device memory of destroyed contexts
+ * and finished gradients (at most a quarter of the device's memory; an
+ * allocation of this library that finds none left frees it too).  They are
+ * allocated again when needed. */
 int lbm_trim(void);
 
 /* Text of the calling thread's last error ("" if none). */

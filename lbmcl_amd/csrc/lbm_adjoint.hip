@@ -5,13 +5,13 @@
 // Schedule for T steps with checkpoints every K steps (M = ceil(T / K)
 // segments):
 //   forward   P_0 -> P_T; P_{mK} is kept for every segment m; the states of
-//             the last segment are kept whole (the tape), so it needs no
-//             recomputation.
+//             the last segments are kept whole (their tapes), as many as memory
+//             is plentiful for, so they need no recomputation.
 //   seed      lambda_T = dJ/dP_T from the objective on the gathered P_T.
 //   reverse   for m = M-1 .. 0: recompute P_{mK+1} .. P_{mK+len-1} from the
-//             checkpoint into the tape (not for the last segment), then step
+//             checkpoint into a tape (not where it is kept), then step
 //             lambda backwards through the segment.
-// Device memory: M checkpoints + (K - 1) tape states + 2 lattices + 2 adjoint
+// Device memory: M checkpoints + (K - 1) states a tape + 2 lattices + 2 adjoint
 // lattices, i.e. about 2 sqrt(T) states for K = sqrt(T).
 // No counterpart in the reference.
 #include <type_traits>
@@ -23,15 +23,18 @@ using namespace lbm_host;
 
 namespace {
 
+// Device memory of one gradient, back in the pool at its end.
 struct AdjointBuffers {
-    std::vector<void*> owned;
+    lbm_ctx* c;
+    std::vector<std::pair<void*, size_t>> owned;
+    explicit AdjointBuffers(lbm_ctx* ctx) : c(ctx) {}
     ~AdjointBuffers() {
-        for (void* p : owned)
-            if (p) (void)hipFree(p);
+        (void)hipStreamSynchronize(c->stream);  // an error may have left work enqueued
+        for (const auto& b : owned) g_pool.give(c->cfg.device, b.first, b.second);
     }
     int alloc(void** p, size_t bytes, const char* what) {
-        const int rc = dev_alloc(p, bytes, what);
-        if (!rc) owned.push_back(*p);
+        const int rc = pool_alloc(c, p, bytes, what);
+        if (!rc) owned.emplace_back(*p, bytes);
         return rc;
     }
 };
@@ -48,6 +51,20 @@ template <class T> int64_t adjoint_vec_width(const lbm_ctx* c) {
     return 0;
 }
 
+// Segments whose states stay on a tape of their own, at least the last one: as
+// many as fit a sixteenth of the device's memory with everything else (18 GB:
+// all of 64^3 FP64 x 150 in 6 GB, 128^3 FP32 up to 110 steps).  Each saves the
+// recomputation of its states, which otherwise is a second forward run.
+int64_t tapes_kept(int64_t segments, int64_t ntape, size_t state) {
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    const int64_t left = int64_t(total / 16 / state) - segments - 4;  // checkpoints, lattices, adjoint lattices
+    return ntape > 0 ? std::max<int64_t>(1, std::min(segments, left / ntape)) : segments;
+}
+
 template <class T>
 int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* res, double* grad_g_host) {
     const int64_t T_steps = cfg.steps;
@@ -57,7 +74,7 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     if (K > T_steps) K = T_steps;
     const int64_t M = (T_steps + K - 1) / K;
     const size_t S = size_t(c->n3) * lbm::Q * sizeof(T);
-    AdjointBuffers buf;
+    AdjointBuffers buf(c);
     double device_bytes = 2.0 * S + double(c->n3) * (4 * sizeof(T) + 4);
 
     // states: ckpt[0] is the context's lattice 0, the final state goes to lattice 1
@@ -68,13 +85,30 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
         if (rc) return rc;
         device_bytes += double(S);
     }
+    // tapes: that of the last segment, which earlier ones recompute their states
+    // into, and one more for each of the `kept` - 1 segments before it
     const int64_t ntape = K - 1;
-    std::vector<void*> tape(size_t(ntape), nullptr);
-    for (int64_t j = 0; j < ntape; ++j) {
-        const int rc = buf.alloc(&tape[size_t(j)], S, "adjoint tape");
-        if (rc) return rc;
-        device_bytes += double(S);
+    int64_t kept = 0;
+    std::vector<void*> tapes;
+    const int64_t want = tapes_kept(M, ntape, S);
+    for (; kept < want; ++kept) {
+        const std::string last_error = g_last_error;
+        int rc = LBM_OK;
+        for (int64_t j = 0; j < ntape && !rc; ++j) {
+            void* p = nullptr;
+            rc = buf.alloc(&p, S, "adjoint tape");
+            tapes.push_back(p);
+        }
+        if (rc && kept == 0) return rc;
+        if (rc) {  // as many as there is memory for
+            g_last_error = last_error;
+            tapes.resize(size_t(kept * ntape));
+            break;
+        }
+        device_bytes += double(S) * double(ntape);
     }
+    const auto is_kept = [&](int64_t m) { return m >= M - kept; };
+    const auto tape_of = [&](int64_t m) { return tapes.data() + (is_kept(m) ? M - 1 - m : 0) * ntape; };
     void* lam[2] = {nullptr, nullptr};
     for (int j = 0; j < 2; ++j) {
         const int rc = buf.alloc(&lam[j], S, "adjoint state");
@@ -132,12 +166,13 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     hipEvent_t evs[3] = {e0, e1, e2};
     EvGuard guard{evs};
 
-    // P_0 in both context lattices, then its wall slots into every other state
+    // P_0 in both context lattices, then its wall slots into every other state:
+    // the rest of them is written by the step that makes the state
     int rc = launch_initialize<T, lbm::ST_NATIVE>(c);
     if (rc) return rc;
-    for (void* p : ckpt)
-        if (p != c->lat[0]) LBM_HIP_CHECK(hipMemcpyAsync(p, c->lat[0], S, hipMemcpyDeviceToDevice, c->stream), "D2D");
-    for (void* p : tape) LBM_HIP_CHECK(hipMemcpyAsync(p, c->lat[0], S, hipMemcpyDeviceToDevice, c->stream), "D2D");
+    rc = launch_walls<T, lbm::ST_NATIVE>(c, ckpt.data() + 1, ckpt.size() - 1);
+    if (!rc) rc = launch_walls<T, lbm::ST_NATIVE>(c, tapes.data(), tapes.size());
+    if (rc) return rc;
 
     // forward with checkpoints
     LBM_HIP_CHECK(hipEventRecord(e0, c->stream), "hipEventRecord");
@@ -145,14 +180,14 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     for (int64_t m = 0; m < M; ++m) {
         const int64_t s0 = m * K;
         const int64_t len = std::min(K, T_steps - s0);
-        const bool last = (m == M - 1);
+        void* const* const tape = tape_of(m);
         const void* src = ckpt[size_t(m)];
         for (int64_t j = 1; j <= len; ++j) {  // produce P_{s0 + j}
             void* dst;
             if (j == len)
-                dst = last ? fin : ckpt[size_t(m + 1)];
+                dst = m == M - 1 ? fin : ckpt[size_t(m + 1)];
             else
-                dst = last ? tape[size_t(j - 1)] : tape[size_t((j - 1) % 2)];
+                dst = is_kept(m) ? tape[j - 1] : tape[(j - 1) % 2];
             rc = launch_compute<T, lbm::ST_NATIVE>(c, src, dst, 0, 0);
             if (rc) return rc;
             src = dst;
@@ -207,16 +242,17 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     for (int64_t m = M - 1; m >= 0; --m) {
         const int64_t s0 = m * K;
         const int64_t len = std::min(K, T_steps - s0);
-        if (m != M - 1) {  // recompute P_{s0+1} .. P_{s0+len-1}
+        void* const* const tape = tape_of(m);
+        if (!is_kept(m)) {  // recompute P_{s0+1} .. P_{s0+len-1}
             const void* src = ckpt[size_t(m)];
             for (int64_t j = 1; j < len; ++j) {
-                rc = launch_compute<T, lbm::ST_NATIVE>(c, src, tape[size_t(j - 1)], 0, 0);
+                rc = launch_compute<T, lbm::ST_NATIVE>(c, src, tape[j - 1], 0, 0);
                 if (rc) return rc;
-                src = tape[size_t(j - 1)];
+                src = tape[j - 1];
             }
         }
         for (int64_t j = len - 1; j >= 0; --j) {  // step k = s0 + j reads P_k
-            const void* Pk = (j == 0) ? ckpt[size_t(m)] : tape[size_t(j - 1)];
+            const void* Pk = (j == 0) ? ckpt[size_t(m)] : tape[j - 1];
             rc = adj_step(Pk, lam[cur], lam[1 - cur], 0, (s0 + j == 0) ? 1 : 0);
             if (rc) return rc;
             cur = 1 - cur;
@@ -262,13 +298,13 @@ int lbm_set_force(lbm_ctx* c, const void* force) {
     if (rc) return rc;
     LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     if (!force) {
-        if (c->force) (void)hipFree(c->force);
+        g_pool.give(c->cfg.device, c->force, size_t(3 * c->n3) * c->tsize);
         c->force = nullptr;
         return LBM_OK;
     }
     const size_t bytes = size_t(3 * c->n3) * c->tsize;
     if (!c->force) {
-        rc = dev_alloc(&c->force, bytes, "body force");
+        rc = pool_alloc(c, &c->force, bytes, "body force");
         if (rc) return rc;
     }
     LBM_HIP_CHECK(hipMemcpyAsync(c->force, force, bytes, hipMemcpyHostToDevice, c->stream), "hipMemcpyAsync H2D");

@@ -115,12 +115,13 @@ int lbm_create(const lbm_config* cfg, lbm_ctx** out) {
     }
     const size_t lat_bytes = size_t(n3) * lbm::Q * c->ssize;
     c->partials_cap = compute_blocks(c);
-    if ((rc = dev_alloc(&c->lat[0], lat_bytes, "lattice 0")) || (rc = dev_alloc(&c->lat[1], lat_bytes, "lattice 1")) ||
-        (rc = dev_alloc(&c->rho, size_t(n3) * c->tsize, "rho")) ||
-        (rc = dev_alloc(&c->u, size_t(3 * n3) * c->tsize, "u")) ||
-        (rc = dev_alloc(reinterpret_cast<void**>(&c->partials), size_t(c->partials_cap) * 2 * sizeof(double),
-                        "partials")) ||
-        (rc = dev_alloc(reinterpret_cast<void**>(&c->diag), 2 * sizeof(double), "diagnostics"))) {
+    if ((rc = pool_alloc(c, &c->lat[0], lat_bytes, "lattice 0")) ||
+        (rc = pool_alloc(c, &c->lat[1], lat_bytes, "lattice 1")) ||
+        (rc = pool_alloc(c, &c->rho, size_t(n3) * c->tsize, "rho")) ||
+        (rc = pool_alloc(c, &c->u, size_t(3 * n3) * c->tsize, "u")) ||
+        (rc = pool_alloc(c, reinterpret_cast<void**>(&c->partials), size_t(c->partials_cap) * 2 * sizeof(double),
+                         "partials")) ||
+        (rc = pool_alloc(c, reinterpret_cast<void**>(&c->diag), 2 * sizeof(double), "diagnostics"))) {
         std::string msg = g_last_error;
         release(c);
         return fail(rc, msg);
@@ -483,6 +484,7 @@ int lbm_kernels_time_ms(lbm_ctx* c, double* ms) {
 }
 
 int lbm_trim(void) {
+    (void)g_pool.trim();
     std::lock_guard<std::mutex> lock(g_pinned.busy);
     g_pinned.free();
     return LBM_OK;

@@ -21,6 +21,7 @@
 
 #include "../../include/lbm_hip.h"
 #include "lbm_kernels.hpp"
+#include "lbm_pool.hpp"
 #include "lbm_slots.hpp"
 #include "lbm_stage.hpp"
 
@@ -241,15 +242,25 @@ inline void release(lbm_ctx* c) {
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
     c->stage.release();
     free_events(c);
-    for (void* p : {c->lat[0], c->lat[1], c->rho, c->u, (void*)c->map, (void*)c->partials, (void*)c->diag, c->force})
-        if (p) (void)hipFree(p);
+    const size_t n3 = size_t(c->n3);
+    for (void* p : c->lat) g_pool.give(c->cfg.device, p, n3 * lbm::Q * c->ssize);
+    g_pool.give(c->cfg.device, c->rho, n3 * c->tsize);
+    g_pool.give(c->cfg.device, c->u, 3 * n3 * c->tsize);
+    g_pool.give(c->cfg.device, c->force, 3 * n3 * c->tsize);
+    g_pool.give(c->cfg.device, c->partials, size_t(c->partials_cap) * 2 * sizeof(double));
+    g_pool.give(c->cfg.device, c->diag, 2 * sizeof(double));
+    if (c->map) (void)hipFree(c->map);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
 
 inline int dev_alloc(void** p, size_t bytes, const char* what) {
     *p = nullptr;
-    const hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        if (g_pool.trim()) e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         *p = nullptr;
         (void)hipGetLastError();
@@ -257,6 +268,13 @@ inline int dev_alloc(void** p, size_t bytes, const char* what) {
                                         " bytes): " + hipGetErrorString(e));
     }
     return LBM_OK;
+}
+
+// dev_alloc from the pool of c's device, which the memory goes back to with
+// g_pool.give once nothing enqueued uses it.
+inline int pool_alloc(const StepPlan* c, void** p, size_t bytes, const char* what) {
+    *p = g_pool.take(c->cfg.device, bytes);
+    return *p ? LBM_OK : dev_alloc(p, bytes, what);
 }
 
 enum KernelKind { K_GENERIC, K_ROW, K_VEC, K_VEC8, K_TILE, K_LDS };
@@ -666,6 +684,22 @@ inline int launch_initialize(lbm_ctx* c) {
     const int64_t nb = (c->n3 + 255) / 256;
     hipLaunchKernelGGL((lbm::lbm_initialize_kernel<T, KIND>), dim3(unsigned(nb)), dim3(256), 0, c->stream, a);
     LBM_HIP_CHECK(hipGetLastError(), "initialize launch");
+    return LBM_OK;
+}
+
+// The wall cells' slots of `count` lattices, as lbm_initialize sets them.
+template <class T, int KIND>
+inline int launch_walls(lbm_ctx* c, void* const* lattices, size_t count) {
+    const lbm::InitArgs<T> a = init_args<T, KIND>(c);
+    const int64_t cells = 6 * int64_t(c->n) * c->n;
+    for (size_t k = 0; k < count; k += lbm::WallTargets::MAX) {
+        lbm::WallTargets t{};
+        const size_t m = std::min<size_t>(lbm::WallTargets::MAX, count - k);
+        std::copy(lattices + k, lattices + k + m, t.lattice);
+        hipLaunchKernelGGL((lbm::lbm_walls_kernel<T, KIND>), dim3(unsigned((cells + 255) / 256), unsigned(m)), dim3(256),
+                           0, c->stream, a, t);
+        LBM_HIP_CHECK(hipGetLastError(), "wall slots launch");
+    }
     return LBM_OK;
 }
 

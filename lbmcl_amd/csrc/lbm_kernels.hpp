@@ -1431,6 +1431,30 @@ __global__ __launch_bounds__(256) void lbm_initialize_kernel(InitArgs<T> a) {
     }
 }
 
+// The slots of the wall cells alone, of several lattices (blockIdx.y): for
+// lattices that a step writes before anything else reads them, which writes
+// every other cell.  A thread per cell of the six faces; the cells that two faces
+// share belong to the first of them (z, then y, then x).
+struct WallTargets {
+    static constexpr int MAX = 64;
+    void* lattice[MAX];
+};
+template <class T, int KIND>
+__global__ __launch_bounds__(256) void lbm_walls_kernel(InitArgs<T> a, WallTargets t) {
+    using S = typename Codec<T, KIND>::S;
+    const int32_t n = a.n;
+    const uint32_t k = blockIdx.x * 256u + threadIdx.x, n2 = uint32_t(n) * uint32_t(n);  // n <= 1024
+    if (k >= 6u * n2) return;
+    const uint32_t face = k / n2;
+    const int32_t u = int32_t(k & uint32_t(n - 1)), v = int32_t((k % n2) >> a.log2n), w = (face & 1u) ? n - 1 : 0;
+    const int32_t x = face < 4 ? u : w, y = face < 2 ? v : (face < 4 ? w : u), z = face < 2 ? w : v;
+    if ((face >= 2 && (z == 0 || z == n - 1)) || (face >= 4 && (y == 0 || y == n - 1))) return;
+    const int64_t c = int64_t(x) + int64_t(n) * (int64_t(y) + int64_t(n) * z);
+    S* const p = static_cast<S*>(t.lattice[blockIdx.y]);
+#pragma unroll
+    for (int i = 0; i < Q; ++i) p[slot(c, i, a.stride)] = initial_slot<T, KIND>(a, i, x, y, z);
+}
+
 // *differ = 1 where a wall cell's slot does not hold its initial value (a NaN
 // stands for any NaN).
 template <class T, int KIND>
