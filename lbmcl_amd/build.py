@@ -54,6 +54,7 @@ OBJ_DIR = os.path.join(PKG, "_build")
 OPENCL_DIVISION = ["-fno-hip-fp32-correctly-rounded-divide-sqrt"]
 LIB_UNITS = {
     "lbm_capi": [], "lbm_adjoint": [], "lbm_noalloc": [], "lbm_two_step": [], "lbm_small": [],
+    "lbm_relayout": [],
     "lbm_opencl_arith": OPENCL_DIVISION, "lbm_two_step_opencl": OPENCL_DIVISION,
     "lbm_small_opencl": OPENCL_DIVISION,
 }

@@ -17,11 +17,22 @@
 #include <type_traits>
 
 #include "lbm_adjoint.hpp"
-#include "lbm_ctx.hpp"
+#include "lbm_range.hpp"
 
 using namespace lbm_host;
 
 namespace {
+
+// The layout of a gradient's states, which nobody else sees: the fastest one
+// where the context's has short runs.
+struct AdjointStride {
+    lbm_ctx* c;
+    const int64_t own;
+    explicit AdjointStride(lbm_ctx* ctx) : c(ctx), own(ctx->stride) {
+        if (relayout_pays(c)) c->stride = kFastStride;
+    }
+    ~AdjointStride() { c->stride = own; }
+};
 
 // Device memory of one gradient, back in the pool at its end.
 struct AdjointBuffers {
@@ -74,6 +85,8 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     if (K > T_steps) K = T_steps;
     const int64_t M = (T_steps + K - 1) / K;
     const size_t S = size_t(c->n3) * lbm::Q * sizeof(T);
+    c->initialized = false;  // the lattices hold no resumable state from here on
+    AdjointStride stride(c);
     AdjointBuffers buf(c);
     double device_bytes = 2.0 * S + double(c->n3) * (4 * sizeof(T) + 4);
 
@@ -284,7 +297,6 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     res->device_bytes = device_bytes;
     res->checkpoints = M;
     res->segment = K;
-    c->initialized = false;  // the lattices no longer hold a resumable state
     return LBM_OK;
 }
 

@@ -44,6 +44,80 @@ int check_walls(lbm_ctx* c, int32_t buffer, bool* same) {
     return rc;
 }
 
+// Iterations [first, first + count) in the plan's layout; `multi`: launches may
+// take several.
+int run_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every, bool multi) {
+    // Without per-launch events, several iterations go in one launch where the
+    // lattice has one (lbm_small.hpp, lbm_two_step.hpp).  Those in between reach
+    // no lattice, so the last one is a launch of its own -- it leaves the last two
+    // states in the two lattices, as iterations one by one do -- except where the
+    // launch itself does that.  The two-step launch stores rho and u of its second
+    // iteration only.
+    const int32_t small = multi ? small_steps(c) : 0;
+    const bool pairs = multi && !small && two_steps_preferred(c);
+    const int64_t end = first + count;
+    for (int64_t it = first; it < end;) {
+        const auto stores = [&](int64_t k) { return every > 0 && k % every == 0 ? 1 : 0; };
+        const int s = (it % 2 != 0) ? 0 : 1;  // the lattice that iteration `it` reads
+        int64_t k = 1;
+        int rc = LBM_OK;
+        if (small && small_is_one_tile(c)) {
+            k = std::min<int64_t>(small, end - it);
+            rc = launch_small(c, c->lat[s], c->lat[(s + k) % 2], k > 1 ? c->lat[(s + k + 1) % 2] : nullptr, int32_t(k),
+                              every, every > 0 ? (it - 1) % every : 0);
+        } else if (small && end - it >= 3) {
+            k = std::min<int64_t>(small, end - it - 1);
+            rc = launch_small(c, c->lat[s], c->lat[1 - s], nullptr, int32_t(k), every, every > 0 ? (it - 1) % every : 0);
+            if (!rc && k % 2 == 0) std::swap(c->lat[0], c->lat[1]);  // the lattice written is the one `it` + k reads
+        } else if (pairs && end - it >= 3 && !stores(it)) {
+            k = 2;
+            rc = launch_two_steps(c, c->lat[s], c->lat[1 - s], stores(it + 1));
+            if (!rc) std::swap(c->lat[0], c->lat[1]);
+        } else {
+            rc = lbm_compute(c, it, stores(it), 0);
+        }
+        if (rc) return rc;
+        it += k;
+    }
+    return LBM_OK;
+}
+
+// The third lattice, if there is room for it: at most an eighth of the device's
+// memory, which a long run on the two lattices can do without.
+bool third_lattice(lbm_ctx* c) {
+    if (c->lat_free) return true;
+    const size_t bytes = size_t(c->n3) * lbm::Q * c->ssize;
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || bytes > total / 8) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const std::string last_error = g_last_error;
+    if (pool_alloc(c, &c->lat_free, bytes, "third lattice")) g_last_error = last_error;
+    return c->lat_free != nullptr;
+}
+
+// run_range in the layout of stride kFastStride: the first iteration's source
+// goes into the third lattice, the other one gets that layout's wall slots, and
+// the last two states come back, each into the lattice that is free by then.
+int run_range_relaid(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
+    const int s = (first % 2 != 0) ? 0 : 1;
+    const int64_t stride = c->stride;
+    int rc = relayout(c, c->lat[s], stride, c->lat_free, kFastStride);
+    if (rc) return rc;
+    std::swap(c->lat[s], c->lat_free);
+    c->stride = kFastStride;
+    rc = LBM_DISPATCH(c, launch_walls, c, &c->lat[1 - s], 1);
+    if (!rc) rc = run_range(c, first, count, every, true);
+    c->stride = stride;
+    for (void*& lattice : c->lat) {
+        if (!rc) rc = relayout(c, lattice, kFastStride, c->lat_free, stride);
+        std::swap(lattice, c->lat_free);
+    }
+    if (rc) c->initialized = false;  // the lattices are in no layout
+    return rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -187,40 +261,10 @@ int lbm_compute_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
     LBM_CHECK_CTX(c);
     LBM_CHECK_INIT(c);
     if (first < 1 || count < 0 || every < 0) return fail(LBM_ERR_INVALID, "bad iteration range");
-    // Without per-launch events, several iterations go in one launch where the
-    // lattice has one (lbm_small.hpp, lbm_two_step.hpp).  Those in between reach
-    // no lattice, so the last one is a launch of its own -- it leaves the last two
-    // states in the two lattices, as iterations one by one do -- except where the
-    // launch itself does that.  The two-step launch stores rho and u of its second
-    // iteration only.
     const bool multi = !c->cfg.profile && c->walls_initial[0] && c->walls_initial[1];
-    const int32_t small = multi ? small_steps(c) : 0;
-    const bool pairs = multi && !small && two_steps_preferred(c);
-    const int64_t end = first + count;
-    for (int64_t it = first; it < end;) {
-        const auto stores = [&](int64_t k) { return every > 0 && k % every == 0 ? 1 : 0; };
-        const int s = (it % 2 != 0) ? 0 : 1;  // the lattice that iteration `it` reads
-        int64_t k = 1;
-        int rc = LBM_OK;
-        if (small && small_is_one_tile(c)) {
-            k = std::min<int64_t>(small, end - it);
-            rc = launch_small(c, c->lat[s], c->lat[(s + k) % 2], k > 1 ? c->lat[(s + k + 1) % 2] : nullptr, int32_t(k),
-                              every, every > 0 ? (it - 1) % every : 0);
-        } else if (small && end - it >= 3) {
-            k = std::min<int64_t>(small, end - it - 1);
-            rc = launch_small(c, c->lat[s], c->lat[1 - s], nullptr, int32_t(k), every, every > 0 ? (it - 1) % every : 0);
-            if (!rc && k % 2 == 0) std::swap(c->lat[0], c->lat[1]);  // the lattice written is the one `it` + k reads
-        } else if (pairs && end - it >= 3 && !stores(it)) {
-            k = 2;
-            rc = launch_two_steps(c, c->lat[s], c->lat[1 - s], stores(it + 1));
-            if (!rc) std::swap(c->lat[0], c->lat[1]);
-        } else {
-            rc = lbm_compute(c, it, stores(it), 0);
-        }
-        if (rc) return rc;
-        it += k;
-    }
-    return LBM_OK;
+    if (multi && count >= kRelayoutRange && relayout_pays(c) && third_lattice(c))
+        return run_range_relaid(c, first, count, every);
+    return run_range(c, first, count, every, multi);
 }
 
 int lbm_finish(lbm_ctx* c) {

@@ -126,6 +126,7 @@ struct StepPlan {
 
 struct lbm_ctx : lbm_host::StepPlan {
     void* lat[2] = {nullptr, nullptr};  // lat[0] read by odd iterations, lat[1] by even
+    void* lat_free = nullptr;           // a third one, for ranges in another layout (allocated by the first)
     // whether the wall cells' slots of each lattice hold the initial lattice's
     // values: so from lbm_initialize on, unless lbm_write_state brought others
     bool walls_initial[2] = {false, false};
@@ -243,7 +244,7 @@ inline void release(lbm_ctx* c) {
     c->stage.release();
     free_events(c);
     const size_t n3 = size_t(c->n3);
-    for (void* p : c->lat) g_pool.give(c->cfg.device, p, n3 * lbm::Q * c->ssize);
+    for (void* p : {c->lat[0], c->lat[1], c->lat_free}) g_pool.give(c->cfg.device, p, n3 * lbm::Q * c->ssize);
     g_pool.give(c->cfg.device, c->rho, n3 * c->tsize);
     g_pool.give(c->cfg.device, c->u, 3 * n3 * c->tsize);
     g_pool.give(c->cfg.device, c->force, 3 * n3 * c->tsize);
