@@ -23,15 +23,19 @@ using namespace lbm_host;
 
 namespace {
 
-// The layout of a gradient's states, which nobody else sees: the fastest one
-// where the context's has short runs.
-struct AdjointStride {
+// How a gradient's steps run: its states, which nobody else sees, are in the
+// fastest layout where the context's has short runs, and are each written once.
+struct AdjointPlan {
     lbm_ctx* c;
     const int64_t own;
-    explicit AdjointStride(lbm_ctx* ctx) : c(ctx), own(ctx->stride) {
+    explicit AdjointPlan(lbm_ctx* ctx) : c(ctx), own(ctx->stride) {
+        c->alternates = false;
         if (relayout_pays(c)) c->stride = kFastStride;
     }
-    ~AdjointStride() { c->stride = own; }
+    ~AdjointPlan() {
+        c->stride = own;
+        c->alternates = true;
+    }
 };
 
 // Device memory of one gradient, back in the pool at its end.
@@ -86,7 +90,7 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     const int64_t M = (T_steps + K - 1) / K;
     const size_t S = size_t(c->n3) * lbm::Q * sizeof(T);
     c->initialized = false;  // the lattices hold no resumable state from here on
-    AdjointStride stride(c);
+    AdjointPlan plan(c);
     AdjointBuffers buf(c);
     double device_bytes = 2.0 * S + double(c->n3) * (4 * sizeof(T) + 4);
 
@@ -183,8 +187,8 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     // the rest of them is written by the step that makes the state
     int rc = launch_initialize<T, lbm::ST_NATIVE>(c);
     if (rc) return rc;
-    rc = launch_walls<T, lbm::ST_NATIVE>(c, ckpt.data() + 1, ckpt.size() - 1);
-    if (!rc) rc = launch_walls<T, lbm::ST_NATIVE>(c, tapes.data(), tapes.size());
+    rc = launch_walls<T, lbm::ST_NATIVE>(c, ckpt.data() + 1, ckpt.size() - 1, true);
+    if (!rc) rc = launch_walls<T, lbm::ST_NATIVE>(c, tapes.data(), tapes.size(), true);
     if (rc) return rc;
 
     // forward with checkpoints

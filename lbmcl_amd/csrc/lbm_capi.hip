@@ -107,7 +107,7 @@ int run_range_relaid(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
     if (rc) return rc;
     std::swap(c->lat[s], c->lat_free);
     c->stride = kFastStride;
-    rc = LBM_DISPATCH(c, launch_walls, c, &c->lat[1 - s], 1);
+    rc = LBM_DISPATCH(c, launch_walls, c, &c->lat[1 - s], 1, false);
     if (!rc) rc = run_range(c, first, count, every, true);
     c->stride = stride;
     for (void*& lattice : c->lat) {

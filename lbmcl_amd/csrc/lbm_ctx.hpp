@@ -120,6 +120,7 @@ struct StepPlan {
     double* partials = nullptr;  // 2 doubles per block of a compute launch (diagnostics)
     void* force = nullptr;       // body force, 3 N^3 of the arithmetic type (null: none)
     double nu = 0, inv_tau = 0, U = 0, scale = 1;
+    bool alternates = true;  // a launch reads the lattice that the one before wrote, and they take turns
 };
 
 }  // namespace lbm_host
@@ -335,6 +336,17 @@ inline bool vec_possible(const StepPlan* c, KernelKind k) {
 // came through LDS.
 inline KernelKind preferred_vec(const StepPlan*) { return K_VEC8; }
 
+// One cell per lane anyway (FP64), and both lattices within half of the last-level
+// cache, each read after it was written: the row kernel, whose loads go through
+// the caches; the vector kernels' streaming loads give their lines up.  64^3 FP64:
+// vector 15.8 us (13.8 with plain loads), row 12.9, generic 13.2.  A gradient's
+// states take no turns, and its forward step is faster with streaming loads, 15.4
+// / 17.6.
+inline bool row_preferred(const StepPlan* c, KernelKind vec) {
+    return lane_bytes(vec) == int64_t(c->ssize) && c->alternates &&
+           2.0 * double(c->n3) * lbm::Q * double(c->ssize) <= 128.0 * 1024 * 1024;
+}
+
 inline KernelKind kernel_kind(const StepPlan* c) {
     switch (c->cfg.kernel) {
         case LBM_KERNEL_GENERIC: return K_GENERIC;
@@ -346,7 +358,7 @@ inline KernelKind kernel_kind(const StepPlan* c) {
         default: {
             if (tile_preferred(c)) return K_TILE;
             const KernelKind p = preferred_vec(c);
-            if (vec_possible(c, p)) return p;
+            if (vec_possible(c, p)) return row_preferred(c, p) ? K_ROW : p;
             if (vec_possible(c, K_VEC8)) return K_VEC8;
             // rows too short for whole wavefronts of vectors (e.g. 16-bit
             // storage below 256^3): the tile kernel when the stride allows it
@@ -368,7 +380,7 @@ inline int64_t row_block(const StepPlan* c) {
     return per_row < 256 ? per_row : 256;
 }
 inline int64_t row_gx(const StepPlan* c) { return (c->n / vec_width(c)) / row_block(c); }
-// Store policy of the 8-byte-lane vector kernel: lattices up to 384 MiB are stored through
+// Store policy of the generic, row and 8-byte-lane vector kernels: lattices up to 384 MiB are stored through
 // the caches, so that much of what a step writes is still in the MI355X's
 // 256 MB memory-attached last-level cache when the next step reads it
 // (measured at 128^3: +13% FP32, +15% FP64); larger ones with streaming
@@ -625,14 +637,19 @@ inline int launch_compute_impl(StepPlan* c, const void* src, void* dst, int upda
                           small_lattice_lds_pad(c, block.x));
             else
                 launch_on(c, lbm::lbm_collide_stream_vec<T, KIND, 8, ARITH, false>, dim3(unsigned(nb)), block, e0, e1, a);
+        } else if (cached_stores(c)) {
+            launch_on(c, lbm::lbm_collide_stream_row<T, KIND, ARITH, true>, dim3(unsigned(nb)), dim3(bx), e0, e1, a);
         } else {
-            launch_on(c, lbm::lbm_collide_stream_row<T, KIND, ARITH>, dim3(unsigned(nb)), dim3(bx), e0, e1, a);
+            launch_on(c, lbm::lbm_collide_stream_row<T, KIND, ARITH, false>, dim3(unsigned(nb)), dim3(bx), e0, e1, a);
         }
     } else {
         const int b = generic_block(c);
         const int64_t nb = (c->n3 + b - 1) / b;
         a.gx = 0;
-        launch_on(c, lbm::lbm_collide_stream_generic<T, KIND, ARITH>, dim3(unsigned(nb)), dim3(b), e0, e1, a);
+        if (cached_stores(c))
+            launch_on(c, lbm::lbm_collide_stream_generic<T, KIND, ARITH, true>, dim3(unsigned(nb)), dim3(b), e0, e1, a);
+        else
+            launch_on(c, lbm::lbm_collide_stream_generic<T, KIND, ARITH, false>, dim3(unsigned(nb)), dim3(b), e0, e1, a);
     }
     LBM_HIP_CHECK(hipGetLastError(), "compute launch");
     return LBM_OK;
@@ -688,13 +705,15 @@ inline int launch_initialize(lbm_ctx* c) {
     return LBM_OK;
 }
 
-// The wall cells' slots of `count` lattices, as lbm_initialize sets them.
+// The wall cells' slots of `count` lattices, as lbm_initialize sets them;
+// read_only: only those that a step reads (64^3 FP64, 64 lattices: 266 us for all).
 template <class T, int KIND>
-inline int launch_walls(lbm_ctx* c, void* const* lattices, size_t count) {
+inline int launch_walls(lbm_ctx* c, void* const* lattices, size_t count, bool read_only) {
     const lbm::InitArgs<T> a = init_args<T, KIND>(c);
     const int64_t cells = 6 * int64_t(c->n) * c->n;
     for (size_t k = 0; k < count; k += lbm::WallTargets::MAX) {
         lbm::WallTargets t{};
+        t.read_only = read_only;
         const size_t m = std::min<size_t>(lbm::WallTargets::MAX, count - k);
         std::copy(lattices + k, lattices + k + m, t.lattice);
         hipLaunchKernelGGL((lbm::lbm_walls_kernel<T, KIND>), dim3(unsigned((cells + 255) / 256), unsigned(m)), dim3(256),
