@@ -176,7 +176,8 @@ int lbm_get_device_name(int32_t device, char* name, size_t len);
  * digits and parsed back as a literal of that type (lbmcl.hpp:140-146). */
 int lbm_create(const lbm_config* config, lbm_ctx** ctx);
 
-/* Release the context and all its device memory (lbmcl.hpp:672-678). */
+/* Release the context and all its device memory (lbmcl.hpp:672-678), which the
+ * library may keep for the next context (lbm_trim). */
 int lbm_destroy(lbm_ctx* ctx);
 
 /* Enqueue the `initialize` kernel (kernels.cl:277-318, lbmcl.hpp:493-498):

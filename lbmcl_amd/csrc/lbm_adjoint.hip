@@ -30,7 +30,7 @@ struct AdjointPlan {
     const int64_t own;
     explicit AdjointPlan(lbm_ctx* ctx) : c(ctx), own(ctx->stride) {
         c->alternates = false;
-        if (relayout_pays(c)) c->stride = kFastStride;
+        if (relayout_possible(c)) c->stride = kFastStride;
     }
     ~AdjointPlan() {
         c->stride = own;

@@ -83,12 +83,15 @@ int run_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every, bool mult
 }
 
 // The third lattice, if there is room for it: at most an eighth of the device's
-// memory, which a long run on the two lattices can do without.
-bool third_lattice(lbm_ctx* c) {
+// memory, which a run on the two lattices can do without.  One too large for the
+// pool is for ranges of 64 iterations or more: the first one may have to wait
+// for memory (10 GB at 512^3 FP32, where an iteration gains 2 ms).
+bool third_lattice(lbm_ctx* c, int64_t count) {
     if (c->lat_free) return true;
     const size_t bytes = size_t(c->n3) * lbm::Q * c->ssize;
     size_t free_bytes = 0, total = 0;
-    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || bytes > total / 8) {
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess ||
+        bytes > total / (count < 64 ? DevicePool::kBlockShare : 8)) {
         (void)hipGetLastError();
         return false;
     }
@@ -262,7 +265,7 @@ int lbm_compute_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
     LBM_CHECK_INIT(c);
     if (first < 1 || count < 0 || every < 0) return fail(LBM_ERR_INVALID, "bad iteration range");
     const bool multi = !c->cfg.profile && c->walls_initial[0] && c->walls_initial[1];
-    if (multi && count >= kRelayoutRange && relayout_pays(c) && third_lattice(c))
+    if (multi && relayout_pays(c, count) && third_lattice(c, count))
         return run_range_relaid(c, first, count, every);
     return run_range(c, first, count, every, multi);
 }

@@ -24,6 +24,8 @@ namespace lbm_host {
 
 class DevicePool {
 public:
+    static constexpr size_t kBlockShare = 64;
+
     // A block of exactly `bytes` of the device, or null.
     void* take(int device, size_t bytes) {
         std::lock_guard<std::mutex> lock(mu_);
@@ -80,7 +82,7 @@ public:
 
 private:
     static constexpr int kMax = 512;
-    static constexpr size_t kShare = 4, kBlockShare = 64;
+    static constexpr size_t kShare = 4;
     struct Block {
         void* p;
         size_t bytes;

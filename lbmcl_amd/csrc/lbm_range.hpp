@@ -13,14 +13,12 @@ int32_t small_steps(const StepPlan* c);
 bool small_is_one_tile(const StepPlan* c);
 int launch_small(StepPlan* c, const void* src, void* dst, void* prev, int32_t k, int64_t every, int64_t phase);
 
-// lbm_relayout.hip: whether iterations are faster in the layout of stride
-// kFastStride than in the plan's own (from 64^3 on: smaller lattices have their
-// own kernel and are read through the caches whole), and a change of a lattice's
-// layout.  Ranges of kRelayoutRange iterations or more are long against the three
-// changes that they take: at 256^3 FP32 stride 16, where an iteration gains least
-// against them, 3 x 0.55 ms against 32 x 0.11.
-constexpr int64_t kFastStride = 4096, kRelayoutRange = 32;
-bool relayout_pays(const StepPlan* c);
+// lbm_relayout.hip: whether a range of `count` iterations is faster in the layout of
+// stride kFastStride than in the plan's own, whether iterations are at all, and a
+// change of a lattice's layout.
+constexpr int64_t kFastStride = 4096;
+bool relayout_possible(const StepPlan* c);
+bool relayout_pays(const StepPlan* c, int64_t count);
 int relayout(lbm_ctx* c, const void* in, int64_t stride_in, void* out, int64_t stride_out);
 
 }  // namespace lbm_host

@@ -54,8 +54,17 @@ __global__ __launch_bounds__(kCells) void relayout_kernel(const U* in, U* out, i
 
 namespace lbm_host {
 
-bool relayout_pays(const StepPlan* c) {
+// From 64^3 on: smaller lattices have their own kernel and are read through the
+// caches whole.
+bool relayout_possible(const StepPlan* c) {
     return c->cfg.kernel == LBM_KERNEL_AUTO && c->n >= 64 && c->stride * int64_t(c->ssize) < 128;
+}
+
+// The three changes cost what 3 to 8 iterations gain with runs of 32 bytes at most
+// (256^3 FP32 stride 1: 3 x 0.55 ms against 0.29 an iteration; 64^3 FP32: 20 us
+// against 4), and up to 15 with longer ones (stride 16: 0.11).
+bool relayout_pays(const StepPlan* c, int64_t count) {
+    return relayout_possible(c) && count >= (c->stride * int64_t(c->ssize) <= 32 ? 12 : 32);
 }
 
 int relayout(lbm_ctx* c, const void* in, int64_t stride_in, void* out, int64_t stride_out) {

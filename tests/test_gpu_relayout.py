@@ -28,7 +28,8 @@ def _agree(a, b):
 
 
 @pytest.mark.parametrize("n, stride, precision, storage, arith, count, every, force", [
-    (64, 1, "f32", "native", "reference", 32, 0, False), (64, 16, "f32", "native", "fused", 33, 5, True),
+    (64, 1, "f32", "native", "reference", 12, 0, False), (64, 4, "f32", "native", "reference", 13, 2, False),
+    (64, 1, "f32", "native", "reference", 11, 0, False), (64, 16, "f32", "native", "reference", 31, 0, False), (64, 16, "f32", "native", "fused", 33, 5, True),
     (64, 4, "f64", "native", "exact", 35, 7, True), (64, 8, "f64", "native", "reference", 32, 1, False),
     (64, 1, "f32", "fp16", "reference", 34, 0, True), (64, 32, "f32", "bf16", "reference", 33, 33, False),
     (128, 2, "f32", "native", "reference", 37, 10, False), (128, 8, "f32", "native", "exact", 32, 0, True),
