@@ -88,6 +88,7 @@ int run_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every, bool mult
 // for memory (10 GB at 512^3 FP32, where an iteration gains 2 ms).
 bool third_lattice(lbm_ctx* c, int64_t count) {
     if (c->lat_free) return true;
+    const AllowAllocation allow;
     const size_t bytes = size_t(c->n3) * lbm::Q * c->ssize;
     size_t free_bytes = 0, total = 0;
     if (hipMemGetInfo(&free_bytes, &total) != hipSuccess ||

@@ -22,6 +22,17 @@
 
 namespace lbm_host {
 
+// For the calling thread: an allocation is allowed while somebody records a HIP
+// graph on a stream of their own, which forbids it to all threads by default and
+// is broken by one.  For allocations in calls that otherwise only launch or copy.
+struct AllowAllocation {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    AllowAllocation() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~AllowAllocation() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    AllowAllocation(const AllowAllocation&) = delete;
+    AllowAllocation& operator=(const AllowAllocation&) = delete;
+};
+
 class DevicePool {
 public:
     static constexpr size_t kBlockShare = 64;

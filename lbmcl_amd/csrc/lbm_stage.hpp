@@ -21,6 +21,8 @@
 #include <mutex>
 #include <thread>
 
+#include "lbm_pool.hpp"
+
 namespace lbm_host {
 
 // The process's pinned buffers, at most HostStage::kBuffers * kChunk (32 MiB),
@@ -34,6 +36,7 @@ struct PinnedBuffers {
 
     hipError_t reserve(size_t bytes) {
         if (bytes <= capacity) return hipSuccess;
+        const AllowAllocation allow;
         free();
         void* p = nullptr;
         const hipError_t rc = hipHostMalloc(&p, bytes, hipHostMallocPortable);

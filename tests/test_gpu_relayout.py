@@ -2,6 +2,8 @@
 the same bits as iterations one by one, in both lattices and in the caller's
 layout, with what may come before and after (a force, an odd first iteration,
 stores, single iterations, a second range)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -63,3 +65,28 @@ def test_written_walls_keep_single_iterations():
             g.compute_range(1, 40, 8)
             out.append([g.read_state(0), g.read_state(1), g.read_rho(), g.read_u()])
     assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(*out))
+
+
+def test_first_range_while_a_graph_is_recorded():
+    """The third lattice is allocated by the first range, which may fall into
+    somebody's recording of a graph on another stream: the recording stays valid."""
+    n = 64
+    capi.lib()
+    h = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library uses
+    stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert h.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0  # non-blocking
+    capi.trim()
+    with capi.Context(n, stride=1, profile=False) as a, capi.Context(n, stride=1, profile=True) as b:
+        for c in (a, b):
+            c.initialize()
+        b.compute_range(1, 40, 8)
+        a.finish()
+        b.finish()
+        assert h.hipStreamBeginCapture(stream, 0) == 0  # global: no thread may allocate
+        try:
+            a.compute_range(1, 40, 8)
+        finally:
+            rc = h.hipStreamEndCapture(stream, ctypes.byref(graph))
+        assert rc == 0 and graph.value
+        assert h.hipGraphDestroy(graph) == 0 and h.hipStreamDestroy(stream) == 0
+        _agree(a, b)
