@@ -8,9 +8,9 @@
 // launch cost more than two launches.  Measured, us per iteration at the stride
 // given / at 4096:
 //   FP32   128^3 stride 1 73 / 35, 8 64 / 35, 16 45 / 35, 32 37 / 35; 256^3 stride 1
-//          557 / 264, 16 373 / 264, 32 275 / 264; 64^3 stride 1 12.4 / 10.2
+//          557 / 264, 16 373 / 264, 32 275 / 264; 64^3 stride 1 12.4 / 8.4
 //   FP64   128^3 stride 1 147 / 68, 4 113 / 68, 8 79 / 68, 16 70 / 68
-//   FP16   128^3 stride 1 48.5 / 31.0, 32 49.5 / 31.0; 256^3 stride 32 294 / 217
+//   FP16   128^3 stride 1 48.5 / 29.0, 32 49.5 / 29.0; 256^3 stride 32 294 / 217
 // Changing the layout reads and writes a lattice once; a range needs it three
 // times (the source, and the last two states), about as long as four
 // iterations.

@@ -11,8 +11,8 @@ namespace lbm_host {
 // widened by 1, 2, 3 / 8 x 4 x 4 by 1, 2 / 8 x 8 x 8 by 1): 16^3 FP32 4.3 / 3.2, 2.7,
 // 2.9 / 3.4, 3.0 / 4.2; 32^3 FP32 4.7 / 3.8, 3.8, 5.6 / 3.6, 3.3 / 5.1, FP64 5.0 / 4.5,
 // 5.6, 6.9 / 4.2, 4.2 / 5.9.  Wider regions take fewer launches but compute more
-// cells twice.  At 64^3 the chip has no idle CUs left for those (FP32 10.2 / 12.8,
-// 15.6, 38 / 10.7, 13.5 / 9.7, FP64 with a force 15.6 / 15.3 at best, FP16 7.7 / 11.2
+// cells twice.  At 64^3 the chip has no idle CUs left for those (FP32 8.4 / 12.8,
+// 15.6, 38 / 10.7, 13.5 / 9.7, FP64 with a force 13.3 / 15.3 at best, FP16 7.7 / 11.2
 // at best): single steps.  8^3: FP32 3.7 / 1.0, FP64 3.9 / 1.4.
 using SmallTile8 = lbm::SmallTile<6, 6, 6, 1>;
 using SmallTile16 = lbm::SmallTile<4, 4, 4, 2>;

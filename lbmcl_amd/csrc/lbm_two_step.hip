@@ -6,7 +6,7 @@ namespace lbm_host {
 
 // Measured on MI355X against the single-step kernels (us per iteration, single /
 // two-step):
-//   lattice   128^3 FP32 48 / 36, FP64 95 / 69; at 64^3 FP32 9.7 / 13.9: too few
+//   lattice   128^3 FP32 48 / 36, FP64 95 / 69; at 64^3 FP32 8.4 / 13.9: too few
 //             planes per block, so not below 128^3
 //   stride    256^3 FP32: 32-byte runs (stride 8) 609 / 515, 16-byte ones 588 /
 //             1143 (the lines of neighbouring populations are then fetched once for
