@@ -67,13 +67,6 @@ __device__ __forceinline__ int lid_multiplicity(int i) {
                                                                    : 1;
 }
 
-// s + e v and e v - s for a component e of a lattice vector, without the products:
-// the compiler may not drop a multiplication by zero, and of the 57 components 27
-// are zero.  The same values.  Reverse step, with the products / without: 256^3
-// FP32 0.73 / 0.69 ms, 128^3 FP32 0.103 / 0.100.
-template <class T> __device__ __forceinline__ T plus_e(T s, int e, T v) { return e > 0 ? s + v : e < 0 ? s - v : s; }
-template <class T> __device__ __forceinline__ T minus_of_e(int e, T v, T s) { return e > 0 ? v - s : e < 0 ? -v - s : -s; }
-
 // Local vector-Jacobian product of one non-wall cell of type t in plane z.
 // f: the populations the cell gathered (the lid fix-up is applied here); L:
 // lambda_{k+1} at the cell's own slots (unused when seeding).  Writes lam
@@ -97,9 +90,9 @@ __device__ __forceinline__ void adjoint_cell(const AdjArgs<T>& a, int32_t t, int
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
         rho += f[i];
-        jx = plus_e(jx, ex_of(i), f[i]);
-        jy = plus_e(jy, ey_of(i), f[i]);
-        jz = plus_e(jz, ez_of(i), f[i]);
+        jx += T(ex_of(i)) * f[i];
+        jy += T(ey_of(i)) * f[i];
+        jz += T(ez_of(i)) * f[i];
     }
     const T ux = jx / rho, uy = jy / rho, uz = jz / rho;
     if (a.seed) {
@@ -151,14 +144,14 @@ __device__ __forceinline__ void adjoint_cell(const AdjArgs<T>& a, int32_t t, int
             A += L[j] * feq;
             const T q = L[j] * rho * w;
             const T k9 = T(9) * eu;
-            Bx += q * minus_of_e(ex_of(j), T(3) + k9, T(3) * ux);
-            By += q * minus_of_e(ey_of(j), T(3) + k9, T(3) * uy);
-            Bz += q * minus_of_e(ez_of(j), T(3) + k9, T(3) * uz);
+            Bx += q * ((T(3) + k9) * T(ex_of(j)) - T(3) * ux);
+            By += q * ((T(3) + k9) * T(ey_of(j)) - T(3) * uy);
+            Bz += q * ((T(3) + k9) * T(ez_of(j)) - T(3) * uz);
             dw += L[j] * (feq - f[j]);
             const double lw = 3.0 * double(L[j]) * double(w);
-            ggx = plus_e(ggx, ex_of(j), lw);
-            ggy = plus_e(ggy, ey_of(j), lw);
-            ggz = plus_e(ggz, ez_of(j), lw);
+            ggx += lw * double(ex_of(j));
+            ggy += lw * double(ey_of(j));
+            ggz += lw * double(ez_of(j));
         }
         A = A / rho;
         const T Bu = Bx * ux + By * uy + Bz * uz;
