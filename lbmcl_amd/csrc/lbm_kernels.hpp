@@ -1471,8 +1471,8 @@ __global__ __launch_bounds__(256) void lbm_walls_kernel(InitArgs<T> a, WallTarge
     }
 }
 
-// *differ = 1 where a wall cell's slot does not hold its initial value (a NaN
-// stands for any NaN).
+// *differ = 1 where a wall cell's slot does not hold the bits of its initial value
+// (a NaN's sign and payload too: a state goes in and comes out as its bytes are).
 template <class T, int KIND>
 __global__ __launch_bounds__(256) void lbm_check_walls_kernel(InitArgs<T> a, const void* lattice, uint32_t* differ) {
     using S = typename Codec<T, KIND>::S;
@@ -1484,15 +1484,11 @@ __global__ __launch_bounds__(256) void lbm_check_walls_kernel(InitArgs<T> a, con
     const int32_t y = int32_t((c >> a.log2n) & (a.n - 1));
     const int32_t z = int32_t(c >> (2 * a.log2n));
     if (!is_wall(cell_type(x, y, z, a.n))) return;
-    const Codec<T, KIND> codec{a.scale, a.inv_scale};
     const S* p = static_cast<const S*>(lattice);
     bool same = true;
 #pragma unroll
-    for (int i = 0; i < Q; ++i) {
-        const S want = initial_slot<T, KIND>(a, i, x, y, z), have = p[slot(c, i, a.stride)];
-        const T w = codec.decode(want, T(0)), h = codec.decode(have, T(0));
-        same = same && (__builtin_bit_cast(U, want) == __builtin_bit_cast(U, have) || (w != w && h != h));
-    }
+    for (int i = 0; i < Q; ++i)
+        same = same && __builtin_bit_cast(U, initial_slot<T, KIND>(a, i, x, y, z)) == __builtin_bit_cast(U, p[slot(c, i, a.stride)]);
     if (!same) *differ = 1;
 }
 
