@@ -11,13 +11,15 @@
 //   reverse   for m = M-1 .. 0: recompute P_{mK+1} .. P_{mK+len-1} from the
 //             checkpoint into a tape (not where it is kept), then step
 //             lambda backwards through the segment.
-// Device memory: M checkpoints + (K - 1) states a tape + 2 lattices + 2 adjoint
-// lattices, i.e. about 2 sqrt(T) states for K = sqrt(T).
+// Device memory: M checkpoints + (K - 1) states of a tape + 2 lattices + 2 adjoint
+// lattices, i.e. about 2 sqrt(T) states for K = sqrt(T), and the tapes that memory
+// is plentiful for (lbm_tapes.hpp): at most all T states.
 // No counterpart in the reference.
 #include <type_traits>
 
 #include "lbm_adjoint.hpp"
 #include "lbm_range.hpp"
+#include "lbm_tapes.hpp"
 
 using namespace lbm_host;
 
@@ -38,10 +40,12 @@ struct AdjointPlan {
     }
 };
 
-// Device memory of one gradient, back in the pool at its end.
+// Device memory of one gradient, back in the pool at its end (allocate_gradient's
+// allocator).
 struct AdjointBuffers {
     lbm_ctx* c;
     std::vector<std::pair<void*, size_t>> owned;
+    size_t free_bytes = 0, total_bytes = 0;
     explicit AdjointBuffers(lbm_ctx* ctx) : c(ctx) {}
     ~AdjointBuffers() {
         (void)hipStreamSynchronize(c->stream);  // an error may have left work enqueued
@@ -52,6 +56,24 @@ struct AdjointBuffers {
         if (!rc) owned.emplace_back(*p, bytes);
         return rc;
     }
+    bool try_alloc(void** p, size_t bytes) {
+        const std::string last_error = g_last_error;
+        if (!alloc(p, bytes, "adjoint tape")) return true;
+        g_last_error = last_error;
+        return false;
+    }
+    void give_back(size_t n) {  // to the device: memory is short
+        for (; n > 0; --n, owned.pop_back()) (void)hipFree(owned.back().first);
+    }
+    size_t available() {
+        if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            free_bytes = total_bytes = 0;
+            return 0;
+        }
+        return free_bytes + g_pool.held(c->cfg.device);
+    }
+    size_t total() const { return total_bytes; }  // as of the last available()
 };
 
 // Cells per lane of the vector adjoint kernel, 0 if it cannot run: it needs
@@ -66,20 +88,6 @@ template <class T> int64_t adjoint_vec_width(const lbm_ctx* c) {
     return 0;
 }
 
-// Segments whose states stay on a tape of their own, at least the last one: as
-// many as fit a sixteenth of the device's memory with everything else (18 GB:
-// all of 64^3 FP64 x 150 in 6 GB, 128^3 FP32 up to 110 steps).  Each saves the
-// recomputation of its states, which otherwise is a second forward run.
-int64_t tapes_kept(int64_t segments, int64_t ntape, size_t state) {
-    size_t free_bytes = 0, total = 0;
-    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
-        (void)hipGetLastError();
-        return 1;
-    }
-    const int64_t left = int64_t(total / 16 / state) - segments - 4;  // checkpoints, lattices, adjoint lattices
-    return ntape > 0 ? std::max<int64_t>(1, std::min(segments, left / ntape)) : segments;
-}
-
 template <class T>
 int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* res, double* grad_g_host) {
     const int64_t T_steps = cfg.steps;
@@ -92,83 +100,48 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     c->initialized = false;  // the lattices hold no resumable state from here on
     AdjointPlan plan(c);
     AdjointBuffers buf(c);
-    double device_bytes = 2.0 * S + double(c->n3) * (4 * sizeof(T) + 4);
-
-    // states: ckpt[0] is the context's lattice 0, the final state goes to lattice 1
-    std::vector<void*> ckpt(size_t(M), nullptr);
-    ckpt[0] = c->lat[0];
-    for (int64_t m = 1; m < M; ++m) {
-        const int rc = buf.alloc(&ckpt[size_t(m)], S, "adjoint checkpoint");
-        if (rc) return rc;
-        device_bytes += double(S);
-    }
-    // tapes: that of the last segment, which earlier ones recompute their states
-    // into, and one more for each of the `kept` - 1 segments before it
-    const int64_t ntape = K - 1;
-    int64_t kept = 0;
-    std::vector<void*> tapes;
-    const int64_t want = tapes_kept(M, ntape, S);
-    for (; kept < want; ++kept) {
-        const std::string last_error = g_last_error;
-        int rc = LBM_OK;
-        for (int64_t j = 0; j < ntape && !rc; ++j) {
-            void* p = nullptr;
-            rc = buf.alloc(&p, S, "adjoint tape");
-            tapes.push_back(p);
-        }
-        if (rc && kept == 0) return rc;
-        if (rc) {  // as many as there is memory for
-            g_last_error = last_error;
-            tapes.resize(size_t(kept * ntape));
-            break;
-        }
-        device_bytes += double(S) * double(ntape);
-    }
-    const auto is_kept = [&](int64_t m) { return m >= M - kept; };
-    const auto tape_of = [&](int64_t m) { return tapes.data() + (is_kept(m) ? M - 1 - m : 0) * ntape; };
-    void* lam[2] = {nullptr, nullptr};
-    for (int j = 0; j < 2; ++j) {
-        const int rc = buf.alloc(&lam[j], S, "adjoint state");
-        if (rc) return rc;
-        device_bytes += double(S);
-    }
-    // dJ/dg: FP64 sum; FP32 runs accumulate in an FP32 buffer flushed into it
-    // every ADJ_FLUSH steps (half the read-modify-write traffic per step)
-    double* grad_g = nullptr;
-    T* grad_acc = nullptr;
     constexpr bool staged = std::is_same<T, float>::value;
-    if (grad_g_host) {
-        const size_t n = size_t(3 * c->n3);
-        int rc = buf.alloc(reinterpret_cast<void**>(&grad_g), n * sizeof(double), "dJ/dg");
-        if (rc) return rc;
-        device_bytes += double(n) * sizeof(double);
-        LBM_HIP_CHECK(hipMemsetAsync(grad_g, 0, n * sizeof(double), c->stream), "hipMemsetAsync");
-        if (staged) {
-            rc = buf.alloc(reinterpret_cast<void**>(&grad_acc), n * sizeof(T), "dJ/dg accumulator");
-            if (rc) return rc;
-            device_bytes += double(n) * sizeof(T);
-            LBM_HIP_CHECK(hipMemsetAsync(grad_acc, 0, n * sizeof(T), c->stream), "hipMemsetAsync");
-        } else {
-            grad_acc = reinterpret_cast<T*>(grad_g);
-        }
-    }
     // vector adjoint kernel: one block of N / V threads per interior row
     const int64_t V = adjoint_vec_width<T>(c);
     const bool vec = V > 0;
     const int block = vec ? int(c->n / V) : 256;
     const int64_t nblocks = vec ? int64_t(c->n - 2) * (c->n - 2) : (c->n3 + 255) / 256;
-    double* partials = nullptr;
-    double* acc = nullptr;
-    {
-        int rc = buf.alloc(reinterpret_cast<void**>(&partials), size_t(3 * nblocks) * sizeof(double), "partials");
-        if (rc) return rc;
-        rc = buf.alloc(reinterpret_cast<void**>(&acc), 3 * sizeof(double), "accumulators");
-        if (rc) return rc;
-        LBM_HIP_CHECK(hipMemsetAsync(partials, 0, size_t(3 * nblocks) * sizeof(double), c->stream), "hipMemsetAsync");
-        LBM_HIP_CHECK(hipMemsetAsync(acc, 0, 3 * sizeof(double), c->stream), "hipMemsetAsync");
-        // slots that no step writes (fed by wall cells) must read as zero
-        for (int j = 0; j < 2; ++j) LBM_HIP_CHECK(hipMemsetAsync(lam[j], 0, S, c->stream), "hipMemsetAsync");
-    }
+
+    GradientSizes z;
+    z.segments = M;
+    z.tape = K - 1;
+    z.state = S;
+    // dJ/dg: FP64 sum; FP32 runs accumulate in an FP32 buffer flushed into it
+    // every ADJ_FLUSH steps (half the read-modify-write traffic per step)
+    z.grad = grad_g_host ? size_t(3 * c->n3) * sizeof(double) : 0;
+    z.grad_stage = grad_g_host && staged ? size_t(3 * c->n3) * sizeof(T) : 0;
+    z.partials = size_t(3 * nblocks) * sizeof(double);
+    z.sums = 3 * sizeof(double);
+    GradientMemory mem;
+    int rc = allocate_gradient(buf, z, &mem);
+    if (rc) return rc;
+    const double device_bytes = double(S) * double(2 + mem.checkpoints.size() + mem.tapes.size() + 2) + double(z.grad) +
+                                double(z.grad_stage) + double(c->n3) * (4 * sizeof(T) + 4);
+
+    // states: ckpt[0] is the context's lattice 0, the final state goes to lattice 1
+    std::vector<void*> ckpt(1, c->lat[0]);
+    ckpt.insert(ckpt.end(), mem.checkpoints.begin(), mem.checkpoints.end());
+    // tapes: that of the last segment, which earlier ones recompute their states
+    // into, and one more for each of the `kept` - 1 segments before it
+    std::vector<void*>& tapes = mem.tapes;
+    const auto is_kept = [&](int64_t m) { return m >= M - mem.kept; };
+    const auto tape_of = [&](int64_t m) { return tapes.data() + (is_kept(m) ? M - 1 - m : 0) * z.tape; };
+    void* const* const lam = mem.lambda;
+    double* const grad_g = static_cast<double*>(mem.grad);
+    T* const grad_acc = static_cast<T*>(staged ? mem.grad_stage : mem.grad);
+    double* const partials = static_cast<double*>(mem.partials);
+    double* const acc = static_cast<double*>(mem.sums);
+    if (grad_g) LBM_HIP_CHECK(hipMemsetAsync(grad_g, 0, z.grad, c->stream), "hipMemsetAsync");
+    if (grad_acc && staged) LBM_HIP_CHECK(hipMemsetAsync(grad_acc, 0, z.grad_stage, c->stream), "hipMemsetAsync");
+    LBM_HIP_CHECK(hipMemsetAsync(partials, 0, z.partials, c->stream), "hipMemsetAsync");
+    LBM_HIP_CHECK(hipMemsetAsync(acc, 0, z.sums, c->stream), "hipMemsetAsync");
+    // slots that no step writes (fed by wall cells) must read as zero
+    for (int j = 0; j < 2; ++j) LBM_HIP_CHECK(hipMemsetAsync(lam[j], 0, S, c->stream), "hipMemsetAsync");
 
     hipEvent_t e0, e1, e2;
     LBM_HIP_CHECK(hipEventCreate(&e0), "hipEventCreate");
@@ -185,7 +158,7 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
 
     // P_0 in both context lattices, then its wall slots into every other state:
     // the rest of them is written by the step that makes the state
-    int rc = launch_initialize<T, lbm::ST_NATIVE>(c);
+    rc = launch_initialize<T, lbm::ST_NATIVE>(c);
     if (rc) return rc;
     rc = launch_walls<T, lbm::ST_NATIVE>(c, ckpt.data() + 1, ckpt.size() - 1, true);
     if (!rc) rc = launch_walls<T, lbm::ST_NATIVE>(c, tapes.data(), tapes.size(), true);

@@ -82,6 +82,14 @@ public:
         blocks_[count_++] = Block{p, bytes, device};
     }
 
+    // Bytes kept of the device.
+    size_t held(int device) {
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t sum = 0;
+        for (int k = 0; k < count_; ++k) sum += blocks_[k].device == device ? blocks_[k].bytes : 0;
+        return sum;
+    }
+
     // Free everything; whether there was anything.
     bool trim() {
         std::lock_guard<std::mutex> lock(mu_);

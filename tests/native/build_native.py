@@ -9,6 +9,7 @@ with sanitizers:
   oracle_selftest   the CPU oracle (oracle/lbm_oracle.cpp): per-slot write
                     counts of the push and pull steps, push == pull, codecs
   slots_test        the snapshot slot state machine (lbmcl_amd/csrc/lbm_slots.hpp)
+  tapes_test        a gradient's device memory (lbmcl_amd/csrc/lbm_tapes.hpp)
 
 sanitize: None, "asan" (-fsanitize=address,undefined, no recovery) or "tsan"
 (-fsanitize=thread).
@@ -35,6 +36,7 @@ PROGRAMS = {
     "lbm_io_selftest": (["lbm_io_selftest.cpp"], ["-pthread"]),
     "oracle_selftest": (["oracle_selftest.cpp"], ["-fopenmp", "-ffp-contract=off", "-fno-fast-math"]),
     "slots_test": (["slots_test.cpp"], ["-pthread"]),
+    "tapes_test": (["tapes_test.cpp"], []),
 }
 
 
