@@ -97,7 +97,6 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     if (K > T_steps) K = T_steps;
     const int64_t M = (T_steps + K - 1) / K;
     const size_t S = size_t(c->n3) * lbm::Q * sizeof(T);
-    c->initialized = false;  // the lattices hold no resumable state from here on
     AdjointPlan plan(c);
     AdjointBuffers buf(c);
     constexpr bool staged = std::is_same<T, float>::value;
@@ -117,6 +116,11 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     z.grad_stage = grad_g_host && staged ? size_t(3 * c->n3) * sizeof(T) : 0;
     z.partials = size_t(3 * nblocks) * sizeof(double);
     z.sums = 3 * sizeof(double);
+    (void)buf.available();
+    if (needed_bytes(z) > double(buf.total()) && buf.total() > 0)
+        return fail(LBM_ERR_MEMORY, "a gradient of " + std::to_string(T_steps) + " steps with a checkpoint every " +
+                                        std::to_string(K) + " needs " + std::to_string(needed_bytes(z) / 1e9) +
+                                        " GB, more than the device has");
     GradientMemory mem;
     int rc = allocate_gradient(buf, z, &mem);
     if (rc) return rc;
@@ -158,6 +162,7 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
 
     // P_0 in both context lattices, then its wall slots into every other state:
     // the rest of them is written by the step that makes the state
+    c->initialized = false;  // the lattices hold no resumable state from here on
     rc = launch_initialize<T, lbm::ST_NATIVE>(c);
     if (rc) return rc;
     rc = launch_walls<T, lbm::ST_NATIVE>(c, ckpt.data() + 1, ckpt.size() - 1, true);

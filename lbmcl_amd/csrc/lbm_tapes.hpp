@@ -27,6 +27,13 @@ struct GradientMemory {
     void *grad = nullptr, *grad_stage = nullptr, *partials = nullptr, *sums = nullptr;
 };
 
+// What the gradient cannot do without, in floating point: it may be more than any
+// device has.
+inline double needed_bytes(const GradientSizes& z) {
+    return (double(z.segments - 1) + double(z.tape) + 2.0) * double(z.state) +
+           double(z.grad + z.grad_stage + z.partials + z.sums);
+}
+
 // Tapes beyond the last segment's.  Each saves the recomputation of its states,
 // which otherwise is a second forward run.  They are for plentiful memory: with all
 // that the gradient holds (`held`, the context's lattices too) they fit a sixteenth

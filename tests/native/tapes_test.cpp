@@ -59,6 +59,7 @@ void run(const lbm_host::GradientSizes& z, size_t capacity, size_t device, size_
     const int rc = allocate_gradient(d, z, &m);
     const size_t needed_blocks = size_t(z.segments - 1 + z.tape + 2 + (z.grad ? 1 : 0) + (z.grad_stage ? 1 : 0) + 2);
     const size_t needed = size_t(z.segments - 1 + z.tape + 2) * z.state + z.grad + z.grad_stage + z.partials + z.sums;
+    check(needed_bytes(z) == double(needed), "needed bytes", long(needed), 0);
     check((rc == 0) == (needed <= capacity && needed_blocks <= blocks), "succeeds where the needed memory fits", long(capacity),
           long(blocks));
     if (rc) return;

@@ -49,3 +49,22 @@ def test_gradient_beside_somebody_elses_memory():
     for k in ("objective", "d_velocity", "d_viscosity"):
         assert got[k] == want[k]
     assert np.array_equal(got["d_force"], want["d_force"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps, every", [(20_000, 1), (100_000_000, 20_000), (10 ** 15, 1)])
+def test_state_survives_a_gradient_without_memory(steps, every):
+    """A gradient that finds no memory has not touched the context's lattices."""
+    n = 64
+    with capi.Context(n, precision="f64", profile=False) as a, capi.Context(n, precision="f64", profile=False) as b:
+        for c in (a, b):
+            c.initialize()
+            c.compute_range(1, 5)
+        with pytest.raises(capi.LbmError) as e:  # 800 GB at least
+            a.adjoint(steps, checkpoint_every=every, grad_force=False)
+        assert e.value.code == capi.LBM_ERR_MEMORY
+        for c in (a, b):
+            c.compute_range(6, 5, 5)
+        for k in (0, 1):
+            assert np.array_equal(a.read_state(k).view(np.uint64), b.read_state(k).view(np.uint64))
+        assert np.array_equal(a.read_rho(), b.read_rho(), equal_nan=True)
