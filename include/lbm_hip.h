@@ -140,7 +140,8 @@ typedef struct lbm_adjoint_config {
     int32_t objective;         /* LBM_OBJECTIVE_* */
     int32_t plane_z;           /* plane of LBM_OBJECTIVE_MEAN_UX_PLANE, 1 .. dim-2 */
     int64_t steps;             /* T: the objective is evaluated on the state after T iterations */
-    int64_t checkpoint_every;  /* K: forward states kept every K steps; 0 = round(sqrt(T)) */
+    int64_t checkpoint_every;  /* K: forward states kept every K steps; 0 = round(sqrt(T)), and more of them
+                                  where memory is plentiful (lbm_adjoint) */
 } lbm_adjoint_config;
 
 #ifdef __cplusplus
@@ -301,7 +302,13 @@ int lbm_set_force(lbm_ctx* ctx, const void* force);
  * return the objective J and its gradients with respect to the lid velocity,
  * the viscosity and (if grad_force is not NULL: 3*dim^3 doubles) the body
  * force, by the adjoint collide-stream step with checkpoints every
- * config->checkpoint_every steps and recomputation of the segments.  Native
+ * config->checkpoint_every steps and recomputation of the segments.  Device
+ * memory for T steps: ceil(T / K) + K states of 19 * dim^3 values beside the
+ * context's lattices, and dJ/dg; with checkpoint_every = 0 the states of as many
+ * segments as fit stay instead of being computed again, while the gradient as a
+ * whole holds at most a sixteenth of the device's memory and half of what is
+ * free stays so.  result->device_bytes says what it was.  A gradient that fails
+ * for want of memory (LBM_ERR_MEMORY) leaves the context as it was.  Native
  * storage only; the arithmetic type of the context is used for the adjoint
  * states, FP64 for the gradient sums.  The context's lattices are left
  * unspecified (call lbm_initialize before computing again).  No counterpart

@@ -12,8 +12,8 @@
 //             checkpoint into a tape (not where it is kept), then step
 //             lambda backwards through the segment.
 // Device memory: M checkpoints + (K - 1) states of a tape + 2 lattices + 2 adjoint
-// lattices, i.e. about 2 sqrt(T) states for K = sqrt(T), and the tapes that memory
-// is plentiful for (lbm_tapes.hpp): at most all T states.
+// lattices, i.e. about 2 sqrt(T) states for K = sqrt(T); and where K is not the
+// caller's, the tapes that memory is plentiful for (lbm_tapes.hpp).
 // No counterpart in the reference.
 #include <type_traits>
 
@@ -116,6 +116,7 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     z.grad_stage = grad_g_host && staged ? size_t(3 * c->n3) * sizeof(T) : 0;
     z.partials = size_t(3 * nblocks) * sizeof(double);
     z.sums = 3 * sizeof(double);
+    z.extra = cfg.checkpoint_every <= 0;
     (void)buf.available();
     if (needed_bytes(z) > double(buf.total()) && buf.total() > 0)
         return fail(LBM_ERR_MEMORY, "a gradient of " + std::to_string(T_steps) + " steps with a checkpoint every " +

@@ -17,6 +17,7 @@ struct GradientSizes {
     size_t grad = 0;           // of the body force's gradient (0: not wanted)
     size_t grad_stage = 0;     // of what it is accumulated in (0: in itself)
     size_t partials = 0, sums = 0;
+    bool extra = true;         // tapes beyond what is needed are wanted
 };
 
 struct GradientMemory {
@@ -35,12 +36,13 @@ inline double needed_bytes(const GradientSizes& z) {
 }
 
 // Tapes beyond the last segment's.  Each saves the recomputation of its states,
-// which otherwise is a second forward run.  They are for plentiful memory: with all
+// which otherwise is a second forward run.  A caller who chose the interval of the
+// checkpoints chose the memory with it and gets none.  They are for plentiful memory: with all
 // that the gradient holds (`held`, the context's lattices too) they fit a sixteenth
 // of the device's (18 GB: all of 64^3 FP64 x 150 in 6 GB, 128^3 FP32 up to 110
 // steps), and they leave half of what is left to others.
 inline int64_t extra_tapes(const GradientSizes& z, size_t held, size_t available, size_t total) {
-    if (z.tape == 0 || z.state == 0) return 0;  // segments of one step need none
+    if (!z.extra || z.tape == 0 || z.state == 0) return 0;  // segments of one step need none
     const size_t share = total / 16 > held ? total / 16 - held : 0;
     const size_t room = std::min(share, available / 2);
     return std::min<int64_t>(z.segments - 1, int64_t(room / (size_t(z.tape) * z.state)));

@@ -75,7 +75,8 @@ void run(const lbm_host::GradientSizes& z, size_t capacity, size_t device, size_
         check(extra * z.state <= (capacity - needed) / 2, "half of what is left stays", long(capacity), long(extra));
         check(2 * z.state + d.used <= device / 16, "a sixteenth of the device's memory", long(d.used), long(device));
     }
-    if (z.tape > 0 && reported == 0 && blocks == SIZE_MAX && m.kept < z.segments) {  // another one would not do
+    check(z.extra || extra == 0, "no tapes that nobody wants", long(extra), 0);
+    if (z.extra && z.tape > 0 && reported == 0 && blocks == SIZE_MAX && m.kept < z.segments) {  // another one would not do
         const size_t more = (extra + size_t(z.tape)) * z.state;
         check(more > (capacity - needed) / 2 || 2 * z.state + needed + more > device / 16, "as many as there is room for",
               long(capacity), long(extra));
@@ -87,11 +88,12 @@ void run(const lbm_host::GradientSizes& z, size_t capacity, size_t device, size_
 int main() {
     for (const int64_t segments : {1, 2, 3, 13})
         for (const int64_t tape : {0, 1, 4, 11})
-            for (const int grad : {0, 1, 2}) {
+            for (const int grad : {0, 1, 2, 3}) {
                 lbm_host::GradientSizes z;
                 z.segments = segments;
                 z.tape = tape;
                 z.state = 1000;
+                z.extra = grad < 3;
                 z.grad = grad > 0 ? 160 : 0;
                 z.grad_stage = grad > 1 ? 80 : 0;
                 z.partials = 48;

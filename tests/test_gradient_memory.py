@@ -52,6 +52,19 @@ def test_gradient_beside_somebody_elses_memory():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n, precision, steps, every, grad", [
+    (32, "f64", 150, 12, True), (32, "f32", 150, 12, False), (64, "f32", 40, 40, True), (64, "f32", 40, 1, True)])
+def test_checkpoint_interval_bounds_the_memory(n, precision, steps, every, grad):
+    """With an interval of the caller's: checkpoints, one tape, two lattices and two
+    adjoint states, and the gradient's buffers."""
+    r = cavity_gradient(n, steps, precision=precision, checkpoint_every=every, grad_force=grad)
+    size = 8 if precision == "f64" else 4
+    states = -(-steps // every) - 1 + every - 1 + 2 + 2
+    fields = (4 * size + 4) + (0 if not grad else 24 + (12 if precision == "f32" else 0))
+    assert r["device_bytes"] == n ** 3 * (states * 19 * size + fields)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("steps, every", [(20_000, 1), (100_000_000, 20_000), (10 ** 15, 1)])
 def test_state_survives_a_gradient_without_memory(steps, every):
     """A gradient that finds no memory has not touched the context's lattices."""
