@@ -44,6 +44,11 @@ int check_walls(lbm_ctx* c, int32_t buffer, bool* same) {
     return rc;
 }
 
+// Whether ranges of the context may take launches that rely on walls_initial.
+bool ranges_need_walls(const lbm_ctx* c) {
+    return !c->cfg.profile && (small_steps(c) || two_steps_possible(c) || relayout_possible(c));
+}
+
 // Iterations [first, first + count) in the plan's layout; `multi`: launches may
 // take several.
 int run_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every, bool multi) {
@@ -446,7 +451,7 @@ int lbm_write_state(lbm_ctx* c, int32_t buffer, const void* in) {
     LBM_HIP_CHECK(hipMemcpyAsync(c->lat[buffer], in, size_t(c->n3) * lbm::Q * c->ssize, hipMemcpyHostToDevice,
                                  c->stream),
                   "hipMemcpyAsync H2D");
-    if (two_steps_possible(c) || small_steps(c)) {
+    if (ranges_need_walls(c)) {
         const int rc = check_walls(c, buffer, &c->walls_initial[buffer]);
         if (rc) return rc;
     }

@@ -129,7 +129,8 @@ struct lbm_ctx : lbm_host::StepPlan {
     void* lat[2] = {nullptr, nullptr};  // lat[0] read by odd iterations, lat[1] by even
     void* lat_free = nullptr;           // a third one, for ranges in another layout (allocated by the first)
     // whether the wall cells' slots of each lattice hold the initial lattice's
-    // bits: so from lbm_initialize on, unless lbm_write_state brought others
+    // bits: so from lbm_initialize on, unless lbm_write_state brought others (which it
+    // looks for where a range could make use of the answer)
     bool walls_initial[2] = {false, false};
     int32_t* map = nullptr;      // cell flags, allocated on first read (ensure_map)
     bool map_valid = false;

@@ -1,5 +1,8 @@
 """States that lbm_write_state brings, and the ranges of iterations that follow: wall
-slots keep their bytes, whatever the launches."""
+slots keep their bytes, whatever the launches, and a restored state takes the
+launches that the run it came from took."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -37,3 +40,46 @@ def test_payloads_of_wall_slots_stay(n, stride, precision, storage, count):
     assert nan.any()
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+def _free_memory():
+    h = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library uses
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert h.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("change", [False, True])
+@pytest.mark.parametrize("n, stride, precision, storage", [
+    (64, 1, "f32", "native"), (64, 4, "f64", "native"), (64, 2, "f32", "fp16"), (128, 2, "f32", "bf16"),
+    (128, 1, "f64", "native"), (128, 8, "f32", "native")])
+def test_restored_states_take_the_fast_layout(n, stride, precision, storage, change):
+    """A range of a restored lattice with short runs allocates the third lattice that
+    the other layout needs, unless a wall slot holds something else than the initial
+    lattice's; the same bits as single iterations in either case."""
+    kw = dict(stride=stride, precision=precision, storage=storage)
+    with capi.Context(n, profile=False, **kw) as a, capi.Context(n, profile=True, **kw) as b:
+        b.initialize()
+        b.compute_range(1, 3)
+        state = [b.read_state(k) for k in (0, 1)]
+        if change:  # cell (0, 3, 5) is a wall; population 1 leaves it for (1, 3, 5)
+            c = n * (3 + n * 5)
+            state[1][((c // stride) * 19 + 1) * stride + c % stride] = state[1][19 * 8]
+        for c in (a, b):
+            c.initialize()
+            for k in (0, 1):
+                c.write_state(k, state[k])
+        capi.trim()
+        a.finish()
+        before = _free_memory()
+        a.compute_range(4, 64, 5)
+        a.finish()
+        taken = before - _free_memory()
+        b.compute_range(4, 64, 5)
+        lattice = 19 * n ** 3 * a.sdtype(0).itemsize
+        assert taken < lattice // 2 if change else taken >= lattice, (taken, lattice)
+        for k in (0, 1):
+            x, y = _words(a.read_state(k)), _words(b.read_state(k))
+            assert np.array_equal(x, y)
+        assert np.array_equal(a.read_rho(), b.read_rho(), equal_nan=True)
+        assert np.array_equal(a.read_u(), b.read_u(), equal_nan=True)
