@@ -215,7 +215,12 @@ int lbm_initialize(lbm_ctx* ctx);
 int lbm_compute(lbm_ctx* ctx, int64_t iteration, int32_t update_macro, int32_t diagnostics);
 
 /* Enqueue iterations first .. first+count-1; update_macro is set on those
- * divisible by `every` when every > 0 (lbmcl.hpp:436). */
+ * divisible by `every` when every > 0 (lbmcl.hpp:436).  A long range on a lattice
+ * with runs (stride times bytes per slot) below 128 bytes may be iterated in
+ * another layout in between, for which the context keeps a third lattice where
+ * memory allows (at most an eighth of the device's, and as much again free) until
+ * lbm_destroy, lbm_trim or an allocation of this library that finds no memory.  A
+ * range that fails may leave the context uninitialised (lbm_initialize). */
 int lbm_compute_range(lbm_ctx* ctx, int64_t first, int64_t count, int64_t every);
 
 /* Block until the stream is idle (queue.finish(), lbmcl.hpp:525-532). */
@@ -338,11 +343,12 @@ int lbm_adjoint(lbm_ctx* ctx, const lbm_adjoint_config* config, lbm_adjoint_resu
 int lbm_compute_noalloc(const lbm_config* cfg, const void* src, void* dst, void* rho, void* u, int32_t update_macro,
                         double* diag, void* stream);
 
-/* Give back what the library keeps between contexts: the pinned buffers of
- * blocking reads (32 MiB at most) and the device memory of destroyed contexts
- * and finished gradients (at most a quarter of the device's memory; an
- * allocation of this library that finds none left frees it too).  They are
- * allocated again when needed. */
+/* Give back what the library keeps: the pinned buffers of blocking reads (32 MiB
+ * at most), the device memory of destroyed contexts and finished gradients (at
+ * most a quarter of the device's memory), and the third lattices of contexts that
+ * are in none of their calls (lbm_compute_range), once the work on them is done.
+ * An allocation of device memory by this library that finds none left does the
+ * same.  They are allocated again when needed. */
 int lbm_trim(void);
 
 /* Text of the calling thread's last error ("" if none). */

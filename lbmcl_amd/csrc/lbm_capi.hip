@@ -87,43 +87,44 @@ int run_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every, bool mult
     return LBM_OK;
 }
 
-// The third lattice, if there is room for it: at most an eighth of the device's
-// memory, which a run on the two lattices can do without.  One too large for the
-// pool is for ranges of 64 iterations or more: the first one may have to wait
-// for memory (10 GB at 512^3 FP32, where an iteration gains 2 ms).
-bool third_lattice(lbm_ctx* c, int64_t count) {
-    if (c->lat_free) return true;
-    const AllowAllocation allow;
+// The third lattice, if there is room for it (null: none).
+void* third_lattice(lbm_ctx* c, int64_t count) {
     const size_t bytes = size_t(c->n3) * lbm::Q * c->ssize;
+    void* p = g_spares.take(c->lat_spare);
+    if (!p) p = g_pool.take(c->cfg.device, bytes);
+    if (p) return p;
+    const AllowAllocation allow;
     size_t free_bytes = 0, total = 0;
-    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess ||
-        bytes > total / (count < 64 ? DevicePool::kBlockShare : 8)) {
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return nullptr;
     }
+    if (!third_lattice_fits(bytes, count, free_bytes, total)) return nullptr;
     const std::string last_error = g_last_error;
-    if (pool_alloc(c, &c->lat_free, bytes, "third lattice")) g_last_error = last_error;
-    return c->lat_free != nullptr;
+    if (dev_alloc(&p, bytes, "third lattice")) g_last_error = last_error;
+    return p;
 }
 
 // run_range in the layout of stride kFastStride: the first iteration's source
 // goes into the third lattice, the other one gets that layout's wall slots, and
 // the last two states come back, each into the lattice that is free by then.
-int run_range_relaid(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
+int run_range_relaid(lbm_ctx* c, int64_t first, int64_t count, int64_t every, void* third) {
     const int s = (first % 2 != 0) ? 0 : 1;
     const int64_t stride = c->stride;
-    int rc = relayout(c, c->lat[s], stride, c->lat_free, kFastStride);
-    if (rc) return rc;
-    std::swap(c->lat[s], c->lat_free);
-    c->stride = kFastStride;
-    rc = LBM_DISPATCH(c, launch_walls, c, &c->lat[1 - s], 1, false);
-    if (!rc) rc = run_range(c, first, count, every, true);
-    c->stride = stride;
-    for (void*& lattice : c->lat) {
-        if (!rc) rc = relayout(c, lattice, kFastStride, c->lat_free, stride);
-        std::swap(lattice, c->lat_free);
+    int rc = relayout(c, c->lat[s], stride, third, kFastStride);
+    if (!rc) {
+        std::swap(c->lat[s], third);
+        c->stride = kFastStride;
+        rc = LBM_DISPATCH(c, launch_walls, c, &c->lat[1 - s], 1, false);
+        if (!rc) rc = run_range(c, first, count, every, true);
+        c->stride = stride;
+        for (void*& lattice : c->lat) {
+            if (!rc) rc = relayout(c, lattice, kFastStride, third, stride);
+            std::swap(lattice, third);
+        }
+        if (rc) c->initialized = false;  // the lattices are in no layout
     }
-    if (rc) c->initialized = false;  // the lattices are in no layout
+    g_spares.park(c->lat_spare, third, c->stream);
     return rc;
 }
 
@@ -271,8 +272,8 @@ int lbm_compute_range(lbm_ctx* c, int64_t first, int64_t count, int64_t every) {
     LBM_CHECK_INIT(c);
     if (first < 1 || count < 0 || every < 0) return fail(LBM_ERR_INVALID, "bad iteration range");
     const bool multi = !c->cfg.profile && c->walls_initial[0] && c->walls_initial[1];
-    if (multi && relayout_pays(c, count) && third_lattice(c, count))
-        return run_range_relaid(c, first, count, every);
+    if (multi && relayout_pays(c, count))
+        if (void* const third = third_lattice(c, count)) return run_range_relaid(c, first, count, every, third);
     return run_range(c, first, count, every, multi);
 }
 
@@ -537,7 +538,7 @@ int lbm_kernels_time_ms(lbm_ctx* c, double* ms) {
 }
 
 int lbm_trim(void) {
-    (void)g_pool.trim();
+    (void)reclaim_memory();
     std::lock_guard<std::mutex> lock(g_pinned.busy);
     g_pinned.free();
     return LBM_OK;

@@ -127,7 +127,7 @@ struct StepPlan {
 
 struct lbm_ctx : lbm_host::StepPlan {
     void* lat[2] = {nullptr, nullptr};  // lat[0] read by odd iterations, lat[1] by even
-    void* lat_free = nullptr;           // a third one, for ranges in another layout (allocated by the first)
+    lbm_host::Spare lat_spare;          // a third one, for ranges in another layout (allocated by the first)
     // whether the wall cells' slots of each lattice hold the initial lattice's
     // bits: so from lbm_initialize on, unless lbm_write_state brought others (which it
     // looks for where a range could make use of the answer)
@@ -246,7 +246,7 @@ inline void release(lbm_ctx* c) {
     c->stage.release();
     free_events(c);
     const size_t n3 = size_t(c->n3);
-    for (void* p : {c->lat[0], c->lat[1], c->lat_free}) g_pool.give(c->cfg.device, p, n3 * lbm::Q * c->ssize);
+    for (void* p : {c->lat[0], c->lat[1], g_spares.take(c->lat_spare)}) g_pool.give(c->cfg.device, p, n3 * lbm::Q * c->ssize);
     g_pool.give(c->cfg.device, c->rho, n3 * c->tsize);
     g_pool.give(c->cfg.device, c->u, 3 * n3 * c->tsize);
     g_pool.give(c->cfg.device, c->force, 3 * n3 * c->tsize);
@@ -262,7 +262,7 @@ inline int dev_alloc(void** p, size_t bytes, const char* what) {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        if (g_pool.trim()) e = hipMalloc(p, bytes);
+        if (reclaim_memory()) e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) {
         *p = nullptr;

@@ -11,8 +11,9 @@
 //
 // Bounds: a block of at most kBlockShare of the device's memory, all of them
 // together at most kShare of it, kMax blocks; beyond that the ones kept longest
-// are freed.  lbm_trim frees all, and so does an allocation of this library that
-// finds no memory.
+// are freed.  lbm_trim frees all, and what contexts keep for themselves between
+// their calls (g_spares), and so does an allocation of this library that finds no
+// memory.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -118,5 +119,61 @@ private:
     size_t total_ = 0;  // the device's memory
 };
 inline DevicePool g_pool;
+
+// Memory that a context keeps between its calls, and that anybody in need may take
+// from it there: an entry is in the list while it is parked.
+struct Spare {
+    void* p = nullptr;
+    hipStream_t stream = nullptr;  // the work that uses it
+    Spare *next = nullptr, *prev = nullptr;
+};
+class SpareList {
+public:
+    void park(Spare& s, void* p, hipStream_t stream) {
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(mu_);
+        s.p = p;
+        s.stream = stream;
+        s.prev = nullptr;
+        s.next = head_;
+        if (head_) head_->prev = &s;
+        head_ = &s;
+    }
+    // What was parked, for the context alone again; null if somebody took it.
+    void* take(Spare& s) {
+        std::lock_guard<std::mutex> lock(mu_);
+        void* const p = s.p;
+        if (p) remove(s);
+        return p;
+    }
+    // Free everything parked; whether there was anything.
+    bool trim() {
+        std::lock_guard<std::mutex> lock(mu_);
+        const bool any = head_ != nullptr;
+        while (head_) {
+            (void)hipStreamSynchronize(head_->stream);
+            (void)hipFree(head_->p);
+            remove(*head_);
+        }
+        return any;
+    }
+
+private:
+    void remove(Spare& s) {
+        if (s.prev) s.prev->next = s.next;
+        else head_ = s.next;
+        if (s.next) s.next->prev = s.prev;
+        s.p = nullptr;
+    }
+    std::mutex mu_;
+    Spare* head_ = nullptr;
+};
+inline SpareList g_spares;
+
+// Free what is kept; whether there was anything.
+inline bool reclaim_memory() {
+    const bool pool = g_pool.trim(), spares = g_spares.trim();
+    return pool || spares;
+}
 
 }  // namespace lbm_host

@@ -19,6 +19,14 @@ int launch_small(StepPlan* c, const void* src, void* dst, void* prev, int32_t k,
 constexpr int64_t kFastStride = 4096;
 bool relayout_possible(const StepPlan* c);
 bool relayout_pays(const StepPlan* c, int64_t count);
+// Whether a third lattice of that size, which a range can do without, may be
+// allocated for one of `count` iterations: at most an eighth of the device's memory,
+// and as much again stays free.  One too large for the pool is for ranges of 64
+// iterations or more: the first one may have to wait for memory (10 GB at 512^3
+// FP32, where an iteration gains 2 ms).
+inline bool third_lattice_fits(size_t bytes, int64_t count, size_t free_bytes, size_t total) {
+    return bytes <= total / (count < 64 ? DevicePool::kBlockShare : 8) && bytes <= free_bytes / 2;
+}
 int relayout(lbm_ctx* c, const void* in, int64_t stride_in, void* out, int64_t stride_out);
 
 }  // namespace lbm_host

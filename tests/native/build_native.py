@@ -10,6 +10,8 @@ with sanitizers:
                     counts of the push and pull steps, push == pull, codecs
   slots_test        the snapshot slot state machine (lbmcl_amd/csrc/lbm_slots.hpp)
   tapes_test        a gradient's device memory (lbmcl_amd/csrc/lbm_tapes.hpp)
+  rules_test        the rules that select launches, from liblbm_hip.so (host code
+                    only, built with hipcc by build_with_library)
 
 sanitize: None, "asan" (-fsanitize=address,undefined, no recovery) or "tsan"
 (-fsanitize=thread).
@@ -50,6 +52,20 @@ def build(name: str, sanitize: str | None = None) -> str:
     cmd = [cxx, "-std=c++17", *opt, "-Wall", "-Wextra", "-I", INCLUDE, "-I", CSRC, "-I", HERE,
            *[os.path.join(HERE, s) for s in sources], *extra, *SANITIZE[sanitize], "-o", out]
     subprocess.run(cmd, check=True)
+    return out
+
+
+def build_with_library(name: str) -> str:
+    """Compile tests/native/<name>.cpp, which includes the library's own headers, as
+    host code against liblbm_hip.so; returns the executable's path."""
+    from lbmcl_amd import build as product
+    os.makedirs(BIN, exist_ok=True)
+    if not os.path.exists(product.LIB):
+        product.build_lib()
+    out = os.path.join(BIN, name)
+    subprocess.run([product.HIPCC, "-x", "hip", *product.HIP_FLAGS, "-O0", "--offload-host-only", "-I", INCLUDE, "-I", CSRC,
+                    os.path.join(HERE, name + ".cpp"), "-o", out, "-L", product.PKG, "-llbm_hip",
+                    "-Wl,-rpath," + product.PKG], check=True, stderr=subprocess.DEVNULL)
     return out
 
 

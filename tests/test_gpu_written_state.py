@@ -1,12 +1,11 @@
 """States that lbm_write_state brings, and the ranges of iterations that follow: wall
 slots keep their bytes, whatever the launches, and a restored state takes the
 launches that the run it came from took."""
-import ctypes
-
 import numpy as np
 import pytest
 
 from lbmcl_amd import capi
+from tests.gpu_memory import free_memory, settled_free_memory
 
 pytestmark = pytest.mark.gpu
 
@@ -42,13 +41,6 @@ def test_payloads_of_wall_slots_stay(n, stride, precision, storage, count):
         assert np.array_equal(a, b)
 
 
-def _free_memory():
-    h = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library uses
-    free, total = ctypes.c_size_t(), ctypes.c_size_t()
-    assert h.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-    return free.value
-
-
 @pytest.mark.parametrize("change", [False, True])
 @pytest.mark.parametrize("n, stride, precision, storage", [
     (64, 1, "f32", "native"), (64, 4, "f64", "native"), (64, 2, "f32", "fp16"), (128, 2, "f32", "bf16"),
@@ -71,13 +63,14 @@ def test_restored_states_take_the_fast_layout(n, stride, precision, storage, cha
                 c.write_state(k, state[k])
         capi.trim()
         a.finish()
-        before = _free_memory()
+        before = settled_free_memory()
         a.compute_range(4, 64, 5)
         a.finish()
-        taken = before - _free_memory()
+        taken = before - free_memory()
         b.compute_range(4, 64, 5)
         lattice = 19 * n ** 3 * a.sdtype(0).itemsize
-        assert taken < lattice // 2 if change else taken >= lattice, (taken, lattice)
+        # a lattice or none; what else the runtime allocates and frees is megabytes
+        assert (taken < lattice // 2) if change else (taken > lattice // 2), (taken, lattice)
         for k in (0, 1):
             x, y = _words(a.read_state(k)), _words(b.read_state(k))
             assert np.array_equal(x, y)

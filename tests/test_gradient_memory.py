@@ -1,7 +1,6 @@
 """A gradient's device memory: what it cannot do without comes first, the tapes that
 save it time only from what is left (CPU: an allocator of a given capacity; GPU:
 somebody else holds most of the memory)."""
-import ctypes
 import os
 import subprocess
 
@@ -10,6 +9,7 @@ import pytest
 
 from lbmcl_amd import capi
 from lbmcl_amd.adjoint import cavity_gradient, gaussian_random_field
+from tests.gpu_memory import memory_held
 from tests.native import build_native
 
 
@@ -26,24 +26,8 @@ def test_gradient_beside_somebody_elses_memory():
     kw = dict(dim=64, steps=150, precision="f64", force=gaussian_random_field(64, 8.0, 1e-6, seed=2))
     want = cavity_gradient(**kw)
     capi.trim()
-    h = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library uses
-    h.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
-    h.hipFree.argtypes = [ctypes.c_void_p]
-    held = []
-    try:
-        while True:
-            free, total = ctypes.c_size_t(), ctypes.c_size_t()
-            assert h.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-            take = min(free.value - (4 << 30), 32 << 30)
-            if take < (64 << 20):
-                break
-            p = ctypes.c_void_p()
-            assert h.hipMalloc(ctypes.byref(p), take) == 0
-            held.append(p)
+    with memory_held(4 << 30):
         got = cavity_gradient(**kw)
-    finally:
-        for p in held:
-            assert h.hipFree(p) == 0
         capi.trim()
     assert got["device_bytes"] < 3e9 < 5e9 < want["device_bytes"]
     for k in ("objective", "d_velocity", "d_viscosity"):
