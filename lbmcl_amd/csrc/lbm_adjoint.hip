@@ -50,6 +50,7 @@ struct AdjointBuffers {
     ~AdjointBuffers() {
         (void)hipStreamSynchronize(c->stream);  // an error may have left work enqueued
         for (const auto& b : owned) g_pool.give(c->cfg.device, b.first, b.second);
+        g_pool.leave_half(c->cfg.device);
     }
     int alloc(void** p, size_t bytes, const char* what) {
         const int rc = pool_alloc(c, p, bytes, what);

@@ -252,6 +252,7 @@ inline void release(lbm_ctx* c) {
     g_pool.give(c->cfg.device, c->force, 3 * n3 * c->tsize);
     g_pool.give(c->cfg.device, c->partials, size_t(c->partials_cap) * 2 * sizeof(double));
     g_pool.give(c->cfg.device, c->diag, 2 * sizeof(double));
+    g_pool.leave_half(c->cfg.device);
     if (c->map) (void)hipFree(c->map);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;

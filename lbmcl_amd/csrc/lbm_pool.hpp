@@ -10,8 +10,8 @@
 // number of steps.
 //
 // Bounds: a block of at most kBlockShare of the device's memory, all of them
-// together at most kShare of it, kMax blocks; beyond that the ones kept longest
-// are freed.  lbm_trim frees all, and what contexts keep for themselves between
+// together at most kShare of it and at most what else is free of it, kMax blocks;
+// beyond that the ones kept longest are freed.  lbm_trim frees all, and what contexts keep for themselves between
 // their calls (g_spares), and so does an allocation of this library that finds no
 // memory.
 #pragma once
@@ -81,6 +81,29 @@ public:
             remove(0);
         }
         blocks_[count_++] = Block{p, bytes, device};
+    }
+
+    // After a give, or several: leave at least as much free as is kept, for other
+    // allocators of the process, which cannot ask for any of this.
+    void leave_half(int device) {
+        size_t free_bytes = 0, total = 0;
+        if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t held = 0;
+        for (int k = 0; k < count_; ++k) held += blocks_[k].device == device ? blocks_[k].bytes : 0;
+        for (int k = 0; k < count_ && held > free_bytes;) {
+            if (blocks_[k].device != device) {
+                ++k;
+                continue;
+            }
+            held -= blocks_[k].bytes;
+            free_bytes += blocks_[k].bytes;
+            (void)hipFree(blocks_[k].p);
+            remove(k);
+        }
     }
 
     // Bytes kept of the device.

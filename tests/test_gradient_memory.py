@@ -9,7 +9,7 @@ import pytest
 
 from lbmcl_amd import capi
 from lbmcl_amd.adjoint import cavity_gradient, gaussian_random_field
-from tests.gpu_memory import memory_held
+from tests.gpu_memory import is_free_soon, memory_held
 from tests.native import build_native
 
 
@@ -33,6 +33,21 @@ def test_gradient_beside_somebody_elses_memory():
     for k in ("objective", "d_velocity", "d_viscosity"):
         assert got[k] == want[k]
     assert np.array_equal(got["d_force"], want["d_force"])
+
+
+@pytest.mark.gpu
+def test_as_much_stays_free_as_is_kept():
+    """What the library keeps after a gradient and after its context is no more than
+    what is free beside it: of 2 GiB, half."""
+    with memory_held(2 << 30):
+        r = cavity_gradient(64, 150, precision="f64")  # 1.5 GB
+        assert r["device_bytes"] > 1.2e9
+        assert is_free_soon(1_000_000_000)
+        with capi.Context(256, stride=4096, profile=False, storage="fp16") as c:  # 1.5 GB, of which the pool has most
+            c.initialize()
+            c.finish()
+        assert is_free_soon(1_000_000_000)
+    capi.trim()
 
 
 @pytest.mark.gpu
