@@ -1,5 +1,5 @@
-// lbm_stage.hpp -- blocking copies from device memory into a caller's pageable
-// memory, through pinned staging buffers.
+// lbm_stage.hpp -- blocking copies from device memory into a caller's memory: where
+// it is pageable, through pinned staging buffers.
 //
 // hipMemcpy into pageable memory moves 10 GB/s on MI355X (the runtime copies
 // through its own staging on one thread, which also takes the page faults of a
@@ -8,6 +8,9 @@
 // the chunks that have arrived while the next ones are on the link.  Measured, 1
 // GiB into fresh pages: 101 ms with hipMemcpy, 75 / 42 / 27 / 25 / 24 ms with 1 / 2
 // / 4 / 6 / 8 threads and chunks of 4 MiB; 4 KiB 22 us with hipMemcpy, 12 us here.
+// Memory that the device reaches itself (a caller's pinned buffer) takes the link's
+// copy without a detour: 1.28 GB in 27.0 ms staged, 22.3 straight; asking the
+// runtime what the pointer is takes a microsecond.
 // The other direction stays with hipMemcpy: its source's pages exist, and it
 // reads them at 25 GB/s (25 MB in 1.0 ms, 4.5 ms this way).
 #pragma once
@@ -82,6 +85,14 @@ struct HostStage {
         return hipSuccess;
     }
 
+    // Whether the device writes to the caller's memory without a staging buffer.
+    static bool reached(const void* host) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, host) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return false;
+    }
+
     // Copy `bytes` of `dev` into `host` behind the work enqueued on `stream`;
     // returns with the bytes in place.  `enqueued` is called once, when every copy
     // is on the stream.
@@ -89,10 +100,10 @@ struct HostStage {
     hipError_t copy(int device, hipStream_t stream, void* host, const void* dev, size_t bytes, F&& enqueued) {
         const size_t chunk = bytes <= kThreadsAbove ? kChunk / 16 : bytes <= 4 * kChunk ? kChunk / 4 : kChunk;
         const int64_t chunks = int64_t((bytes + chunk - 1) / chunk);
-        std::unique_lock<std::mutex> lock(g_pinned.busy, std::try_to_lock);
-        if (!lock || create_events() != hipSuccess ||
+        std::unique_lock<std::mutex> lock(g_pinned.busy, std::defer_lock);
+        if (reached(host) || !lock.try_lock() || create_events() != hipSuccess ||
             g_pinned.reserve(kBuffers * (bytes <= kThreadsAbove ? kChunk / 16 : kChunk)) != hipSuccess) {
-            (void)hipGetLastError();  // no pinned buffers: as the runtime does it
+            (void)hipGetLastError();  // no need of pinned buffers, or none: as the runtime does it
             const hipError_t rc = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream);
             enqueued();
             const hipError_t rs = hipStreamSynchronize(stream);

@@ -10,6 +10,8 @@ with sanitizers:
                     counts of the push and pull steps, push == pull, codecs
   slots_test        the snapshot slot state machine (lbmcl_amd/csrc/lbm_slots.hpp)
   tapes_test        a gradient's device memory (lbmcl_amd/csrc/lbm_tapes.hpp)
+  stage_test        blocking reads (lbmcl_amd/csrc/lbm_stage.hpp) on a HIP runtime of
+                    host threads (tests/native/host_hip)
   rules_test        the rules that select launches, from liblbm_hip.so (host code
                     only, built with hipcc by build_with_library)
 
@@ -39,6 +41,7 @@ PROGRAMS = {
     "oracle_selftest": (["oracle_selftest.cpp"], ["-fopenmp", "-ffp-contract=off", "-fno-fast-math"]),
     "slots_test": (["slots_test.cpp"], ["-pthread"]),
     "tapes_test": (["tapes_test.cpp"], []),
+    "stage_test": (["stage_test.cpp"], ["-pthread", "-I", os.path.join(HERE, "host_hip")]),
 }
 
 
