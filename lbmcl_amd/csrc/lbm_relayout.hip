@@ -60,11 +60,18 @@ bool relayout_possible(const StepPlan* c) {
     return c->cfg.kernel == LBM_KERNEL_AUTO && c->n >= 64 && c->stride * int64_t(c->ssize) < 128;
 }
 
-// The three changes cost what 3 to 8 iterations gain with runs of 32 bytes at most
-// (256^3 FP32 stride 1: 3 x 0.55 ms against 0.29 an iteration; 64^3 FP32: 20 us
-// against 4), and up to 15 with longer ones (stride 16: 0.11).
+// Where the three changes have paid for themselves: the fixed cost of a relaid range
+// over what an iteration gains, the worst of storing rho and u never, every second
+// and every iteration, with and without a force (which decide whether two steps go
+// in one launch in either layout).  Measured, iterations at 64^3 / 128^3 / 256^3 / 512^3:
+//   runs of at most 32 bytes    FP32 11 / 9 / 9 / 10, FP64 7 / 12 / 10, 16-bit 20 / 5 / 7
+//   runs of 64 bytes            FP32 8 / 20 / 29 / 15, FP64 60 / 56 / 45 / 77, 16-bit 15 / 5 / 11 / 9
+// (64^3 16-bit gains 2 us an iteration for 30, 64^3 FP64 with runs of 64 bytes 1 for
+// 50, 128^3 11 for 450, 512^3 370 for 28000.)
 bool relayout_pays(const StepPlan* c, int64_t count) {
-    return relayout_possible(c) && count >= (c->stride * int64_t(c->ssize) <= 32 ? 12 : 32);
+    if (!relayout_possible(c)) return false;
+    if (c->stride * int64_t(c->ssize) <= 32) return count >= (c->ssize == 2 && c->n == 64 ? 24 : 12);
+    return count >= (c->ssize == 8 ? 96 : 32);
 }
 
 int relayout(lbm_ctx* c, const void* in, int64_t stride_in, void* out, int64_t stride_out) {

@@ -57,3 +57,20 @@ def test_another_allocation_takes_it_back():
             a.compute_range(41, 40, 7)
             _agree(a, b)
     capi.trim()
+
+
+@pytest.mark.parametrize("n, stride, precision, storage, from_", [
+    (64, 8, "f64", "native", 96), (64, 1, "f32", "fp16", 24), (64, 16, "f32", "bf16", 24)])
+def test_ranges_about_the_length_that_pays(n, stride, precision, storage, from_):
+    """One iteration less stays in the layout, one more goes through the other: the
+    same bits as single iterations."""
+    kw = dict(stride=stride, precision=precision, storage=storage, velocity=0.07)
+    for count in (from_ - 1, from_, from_ + 1):
+        with capi.Context(n, profile=False, **kw) as a, capi.Context(n, profile=True, **kw) as b:
+            for c in (a, b):
+                c.initialize()
+                c.compute_range(1, count, 5)
+            for k in (0, 1):
+                assert np.array_equal(a.read_state(k).view(np.uint8), b.read_state(k).view(np.uint8))
+            assert np.array_equal(a.read_rho(), b.read_rho(), equal_nan=True)
+            assert np.array_equal(a.read_u(), b.read_u(), equal_nan=True)
