@@ -41,6 +41,7 @@ template <class T> inline int32_t two_step_segment(int32_t n) {
 
 template <class T, int KIND, int ARITH>
 inline int launch_two_steps_impl(StepPlan* c, const void* src, void* dst, int macro_last) {
+    if (sizeof(T) == 4 && c->force) return fail(LBM_ERR_INVALID, "no two-step launch in FP32 with a force");
     constexpr int threads = lbm::TwoStepThreads<T>::value;
     lbm::TwoStepArgs<T> a{};
     a.s = step_args<T, ARITH>(c, src, dst, 0, 0);

@@ -72,9 +72,29 @@ void other_layout() {
     }
 }
 
+// A launch that no kernel was built for is an error, not a success without a launch
+// (FP32 with a force, refused before the device is asked for anything).
+void launches_without_a_kernel() {
+    double force = 0;
+    for (const int arith : {LBM_ARITH_OPENCL, LBM_ARITH_FUSED, LBM_ARITH_EXACT}) {
+        lbm_config c = LBM_CONFIG_INIT;
+        c.dim = 128;
+        c.stride = 4096;
+        c.viscosity = 0.01;
+        c.velocity = 0.05;
+        c.optimize = arith;
+        StepPlan plan;
+        check(plan_from_config(c, &plan) == LBM_OK && two_steps_preferred(&plan), "a plan for two steps", arith);
+        plan.force = &force;
+        check(!two_steps_preferred(&plan), "single steps with a force", arith);
+        check(launch_two_steps(&plan, nullptr, nullptr, 0) == LBM_ERR_INVALID, "no two-step launch with a force", arith);
+    }
+}
+
 }  // namespace
 
 int main() {
+    launches_without_a_kernel();
     other_layout();
     third_lattices();
     if (failures) return 1;
