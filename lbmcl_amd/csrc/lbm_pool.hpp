@@ -25,7 +25,8 @@ namespace lbm_host {
 
 // For the calling thread: an allocation is allowed while somebody records a HIP
 // graph on a stream of their own, which forbids it to all threads by default and
-// is broken by one.  For allocations in calls that otherwise only launch or copy.
+// is broken by one.  For allocations in calls that otherwise only launch; those that
+// wait for a stream (reads, lbm_finish) the runtime refuses then in any case.
 struct AllowAllocation {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     AllowAllocation() { (void)hipThreadExchangeStreamCaptureMode(&mode); }

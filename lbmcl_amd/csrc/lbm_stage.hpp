@@ -39,7 +39,6 @@ struct PinnedBuffers {
 
     hipError_t reserve(size_t bytes) {
         if (bytes <= capacity) return hipSuccess;
-        const AllowAllocation allow;
         free();
         void* p = nullptr;
         const hipError_t rc = hipHostMalloc(&p, bytes, hipHostMallocPortable);
