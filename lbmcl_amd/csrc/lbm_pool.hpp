@@ -3,9 +3,11 @@
 // hipMalloc and hipFree of a gradient's states cost more than the gradient: the
 // driver clears memory that was freed before it hands it out again, at about 60
 // GB/s, so a program that computes one gradient after another waits for that.
-// Measured, calls one after another: 256^3 FP32 x 200 (40 GB of states) 1008 ms
-// a call, of which the kernels are 310, and 323 with this; 64^3 FP64 x 150 (1.1
-// GB) 17.3 ms, and 8.2 with this and a tape of all states.  Freed blocks are kept
+// Measured on several hosts, which differ in how long the driver takes, calls one
+// after another without the pool / with it: 256^3 FP32 x 200 (40 GB of states, 310
+// ms of kernels) 376 to 1008 ms / 320; 64^3 FP64 x 150 17.3 to 17.9 / 7.4, with a
+// tape of all states.  The first call of a process has no pool yet: 393 / 334 and
+// 27.4 / 22.6 (other memory, and the tapes).  Freed blocks are kept
 // here and given out again by their exact size, which is that of a state for any
 // number of steps.
 //
