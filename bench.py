@@ -3,18 +3,17 @@
 
 Workload: the 512^3 cavity (nu = 0.0089, lid u = 0.05), FP32 populations in
 the CSoA layout with stride 4096 (the fastest stride measured on MI355X: 16 KB
-runs of each population; stride 64 is ~5% slower), the vector row kernel
-(8-byte lanes), the default arithmetic (lbm_config.optimize = 0): kernels.cl's
-expressions as ROCm's OpenCL compiler evaluates them, i.e. the reference's
-results bit for bit.  A "step" is one collide-stream iteration of the
+runs of each population; stride 64 is ~5% slower), the default arithmetic
+(lbm_config.optimize = 0): kernels.cl's expressions as ROCm's OpenCL compiler
+evaluates them, i.e. the reference's results bit for bit.  A "step" is one collide-stream iteration of the
 whole lattice.  The timed region
 holds exactly --steps iterations enqueued back to back on the library's stream,
 bracketed by device synchronisation; the lattice is resident in HBM and already
 initialised before it starts.  Without per-launch events the library advances
 two iterations per launch where the lattice has such a kernel (native storage
-from 128^3 on): `value`, `mlups` and `ms_per_step` are of those; with events
-every iteration is a launch of its own, which is what `kernel_mlups` and the
-roofline time.
+from 128^3 on): `value`, `mlups` and `ms_per_step` are of those (lbm_two_steps);
+with events every iteration is a launch of its own of the vector row kernel
+(8-byte lanes), which is what `kernel_mlups` and the roofline time.
 
 Printed: one JSON line with MLUPS (the reference's definition,
 (dim-2)^3 * iterations / time, lbmcl.hpp:601-620), the HBM roofline of the
@@ -284,6 +283,8 @@ def main():
         cpu = cpu_baseline(dim, args.cpu_steps, args.cpu_threads, stride)
 
     wet = (dim - 2) ** 3
+    two = dim >= 128 and args.kernel == 0 and 4 * stride >= 32  # value's launches (the roofline's are single steps)
+    launches = "two iterations a launch" if two else "single steps"
     traffic = traffic_from_profiles(dim, stride, "f32", "native")
     out = {
         "metric": f"MLUPS (D3Q19 lid-driven cavity, {dim}^3, FP32)",
@@ -299,7 +300,7 @@ def main():
         "dtype": "f32",
         "data": "synthetic (deterministic lid-driven cavity initial state; no dataset)",
         "config": {"workload": f"D3Q19 BGK lid-driven cavity {dim}^3, nu=0.0089, lid u=0.05, FP32 populations, "
-                               f"CSoA stride {stride}, pull-form vector row kernel, the reference's arithmetic "
+                               f"CSoA stride {stride}, pull form, {launches}, the reference's arithmetic "
                                "(kernels.cl as ROCm's OpenCL compiler evaluates it; lbm_config.optimize = 0)",
                    "dim": dim, "stride": stride, "wet_cells": wet, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(main_run["achieved_gbs"], 1), "peak": HBM_PEAK_GBS,
@@ -308,6 +309,7 @@ def main():
                      "traffic_profile": {"file": "profiles/" + traffic[1], "kernel_sources_sha": traffic[2],
                                          "current_sources_sha": kernel_sources_sha()},
                      "kernel": "lbm_collide_stream_vec<float, native, 8-byte lanes, OpenCL arithmetic>",
+                     "timed": "single steps, one launch an iteration with per-launch events (kernel_mlups)",
                      "avg_kernel_ms": round(main_run["avg_kernel_ms"], 4),
                      "bytes_per_launch": wet * 152},
         "cpu_baseline": cpu,

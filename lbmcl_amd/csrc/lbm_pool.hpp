@@ -13,9 +13,9 @@
 //
 // Bounds: a block of at most kBlockShare of the device's memory, all of them
 // together at most kShare of it and at most what else is free of it, kMax blocks;
-// beyond that the ones kept longest are freed.  lbm_trim frees all, and what contexts keep for themselves between
-// their calls (g_spares), and so does an allocation of this library that finds no
-// memory.
+// beyond that the ones kept longest are freed.  lbm_trim frees all, and what
+// contexts keep for themselves between their calls (g_spares), and so does an
+// allocation of this library that finds no memory.
 #pragma once
 
 #include <hip/hip_runtime.h>

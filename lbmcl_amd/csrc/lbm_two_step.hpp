@@ -35,12 +35,16 @@
 // initial population of the cell it arrives at -- the lid layer's equilibrium
 // in the plane N - 2, w_i below it.
 //
-// What bounds it: memory.  Measured at 512^3, FP32, stride 4096: 2.09 ms per
-// iteration against 3.28 for the single step, the same without the arithmetic
-// (2.0), 1.05 with the arithmetic alone.  A pair moves 2.10e10 bytes (1.04 times
-// one read and one write of the lattice) at 5.0 TB/s, where the single step
-// moves 6.2: the tile's rows are loaded by two blocks, which share them through
-// L2.  Prefetching two planes instead of one gains nothing (2.07 without the
+// What bounds it: on large lattices in FP32 memory, with arithmetic not far behind;
+// at 128^3 and in FP64 a round's latency.  Measured at 512^3, FP32, stride 4096:
+// 2.09 ms per iteration against 3.28 for the single step, the same without the
+// arithmetic (2.0), 1.05 with the arithmetic alone; the VALU is busy 0.74 of the
+// time.  A pair moves 2.10e10 bytes (1.04 times one read and one write of the
+// lattice) at 5.0 TB/s, where the single step moves 6.2: the tile's rows are loaded
+// by two blocks, which share them through L2.  128^3, stride 64: FP32 37 us an
+// iteration at 4.8 TB/s with the VALU busy 0.59 of the time, FP64 69 us at 4.7 TB/s
+// and 0.35 -- a plane's loads, LDS and barrier follow one another, and two
+// wavefronts per SIMD (FP64) hide little of it.  Prefetching two planes instead of one gains nothing (2.07 without the
 // arithmetic); tiles whose rows are not whole aligned 256-byte pieces lose most
 // of the gain (3.4 ms).  FP64: 4.35 against 6.6 ms.
 #pragma once
