@@ -345,7 +345,8 @@ int lbm_compute_noalloc(const lbm_config* cfg, const void* src, void* dst, void*
 
 /* Give back what the library keeps: the pinned buffers of blocking reads (32 MiB
  * at most), the device memory of destroyed contexts and finished gradients (at
- * most a quarter of the device's memory, and no more than was free beside it), and the third lattices of contexts that
+ * most a quarter of the device's memory, and beyond 1/256 of it no more than was
+ * free beside them), and the third lattices of contexts that
  * are in none of their calls (lbm_compute_range), once the work on them is done.
  * An allocation of device memory by this library that finds none left does the
  * same.  They are allocated again when needed. */

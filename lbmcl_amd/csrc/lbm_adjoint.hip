@@ -118,8 +118,8 @@ int run_adjoint(lbm_ctx* c, const lbm_adjoint_config& cfg, lbm_adjoint_result* r
     z.partials = size_t(3 * nblocks) * sizeof(double);
     z.sums = 3 * sizeof(double);
     z.extra = cfg.checkpoint_every <= 0;
-    (void)buf.available();
-    if (needed_bytes(z) > double(buf.total()) && buf.total() > 0)
+    const size_t memory = g_pool.device_memory();
+    if (memory > 0 && needed_bytes(z) > double(memory))
         return fail(LBM_ERR_MEMORY, "a gradient of " + std::to_string(T_steps) + " steps with a checkpoint every " +
                                         std::to_string(K) + " needs " + std::to_string(needed_bytes(z) / 1e9) +
                                         " GB, more than the device has");

@@ -42,7 +42,7 @@ inline double needed_bytes(const GradientSizes& z) {
 // of the device's (18 GB: all of 64^3 FP64 x 150 in 6 GB, 128^3 FP32 up to 110
 // steps), and they leave half of what is left to others.
 inline int64_t extra_tapes(const GradientSizes& z, size_t held, size_t available, size_t total) {
-    if (!z.extra || z.tape == 0 || z.state == 0) return 0;  // segments of one step need none
+    if (!z.extra || z.tape == 0) return 0;  // segments of one step need none
     const size_t share = total / 16 > held ? total / 16 - held : 0;
     const size_t room = std::min(share, available / 2);
     return std::min<int64_t>(z.segments - 1, int64_t(room / (size_t(z.tape) * z.state)));
@@ -69,7 +69,8 @@ template <class A> int allocate_gradient(A& a, const GradientSizes& z, GradientM
     if (!rc) rc = needed(&m->sums, z.sums, "accumulators");
     if (rc) return rc;
     m->kept = 1;
-    const int64_t extra = extra_tapes(z, held, a.available(), a.total());
+    const size_t available = z.extra && z.tape > 0 ? a.available() : 0;  // before total()
+    const int64_t extra = extra_tapes(z, held, available, a.total());
     m->tapes.reserve(size_t((1 + extra) * z.tape));
     while (m->kept < 1 + extra) {
         int64_t got = 0;
